@@ -32,10 +32,11 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <tuple>
 #include <vector>
 
-#include "ohm_precond.h"
+#include "ohm_persist.h"
 #include "ohm_reduce.h"
 #include "ohm_sources.h"
 
@@ -2580,6 +2581,7 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
     }
     SegWord *hw = reinterpret_cast<SegWord *>(b->h_pinned);
     *hw = SegWord{0, 0, 0, (int)n_rec, 0, 0, 0, t};
+    auto resident = std::make_unique<ResidentGuard>(true);  // the segment may hold resident solves
     if ((rc = OHM_HIP_STATUS(hipMemcpyAsync(tr->d_seg, hw, sizeof(SegWord), hipMemcpyHostToDevice,
                                        stream))) != OHM_OK ||
         (rc = OHM_HIP_STATUS(hipGraphLaunch(exec, stream))) != OHM_OK ||
@@ -2588,6 +2590,7 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
         (rc = OHM_HIP_STATUS(hipStreamSynchronize(stream))) != OHM_OK)
       return false;
     b->readbacks++;
+    resident.reset();
     const SegWord w = *hw;
     for (int j = 0; j < w.steps; j++) {  // accepted steps: the host's own clock
       t = ts[j];

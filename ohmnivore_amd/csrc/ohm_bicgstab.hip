@@ -25,12 +25,17 @@
 // when the product is formed, else M_L followed by an M_U launch). The same
 // kernels run in FP32 (with compensated dot products) as the inner solver of
 // FP64 iterative refinement.
+//
+// Systems of up to 512 rows per compute unit with short rows take the
+// resident solve instead (ohm_persist.hip: K1-K5 in one launch, behind the
+// same start); a check_interval of the caller's own keeps the pipeline, whose
+// chunks it sizes.
 #include <algorithm>
 #include <cstddef>
 #include <cmath>
 #include <mutex>
 
-#include "ohm_precond.h"
+#include "ohm_persist.h"
 #include "ohm_spmv.h"
 
 namespace ohm {
@@ -193,7 +198,8 @@ __host__ __device__ inline double forcing_eta(const Forcing &fc, double f) {
 }
 
 // r = b - A x0 (warm) or b; r_hat = hashed or r; p = v = 0; x = 0 (cold).
-// Also leaves the r.r / r_hat.r partials where the first p update reads them.
+// Also leaves the r.r / r_hat.r partials where the first p update reads them,
+// and clears the words of a resident solve that follows.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_init(int n, const T *__restrict__ b,
                                                  const T *__restrict__ ax0, T *__restrict__ x,
@@ -202,8 +208,11 @@ __global__ __launch_bounds__(kBlock) void k_init(int n, const T *__restrict__ b,
                                                  int warm, double tol, double floor_rel,
                                                  int tol_mode, int max_iters, int scaled,
                                                  Forcing fc, SolveState *st, Parts pp,
-                                                 int masked) {
+                                                 int masked, uint64_t *clear,
+                                                 int64_t clear_words) {
   if (masked && st->status != ST_RUNNING) return;  // a masked-off captured solve
+  for (int64_t i = blockIdx.x * kBlock + threadIdx.x; i < clear_words; i += gridDim.x * kBlock)
+    clear[i] = 0;
   Acc<T> bb, rr, rhr, hh;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
     T bi = b[i];
@@ -772,6 +781,8 @@ struct Workspace {
   SolveState *st = nullptr;
   BicgVecs<T> v{};
   double *partials = nullptr;  // null: the backend's partials buffer
+  void *resident = nullptr;    // null: the backend's resident workspace
+  size_t resident_bytes = 0;
 };
 
 static Workspace<double> g_ws64;  // one cached workspace per type (single-threaded backend)
@@ -1039,6 +1050,14 @@ static_assert(offsetof(SolveState, r0) - offsetof(SolveState, status) ==
                   sizeof(SolveState) - offsetof(SolveState, status) == sizeof(StatusWord),
               "StatusWord mirrors the tail of SolveState");
 
+static void bicg_out(const StatusWord *h, BicgOut &out) {
+  out.status = h->status;
+  out.iters = h->iters;
+  out.r0 = h->r0;
+  out.res = sqrt(h->res2);
+  out.eta = h->eta;
+}
+
 // Enqueues the start of a solve on the workspace vectors: state reset, the
 // warm-start product A x0 and k_init (rhs is a separate device vector; x0 is
 // read from w.v.x). With stop set (captured solves) the solve is masked off
@@ -1046,7 +1065,8 @@ static_assert(offsetof(SolveState, r0) - offsetof(SolveState, status) ==
 template <typename T>
 static ohm_status bicg_start(ohm_backend *b, const DevCsr &a, const PrecondDev &p, const T *rhs,
                              Workspace<T> &w, const BicgOpts &o, Parts &pp,
-                             const int *stop = nullptr) {
+                             const int *stop = nullptr, void *clear = nullptr,
+                             size_t clear_words = 0) {
   const int n = a.n;
   SolveState *st = w.st;
   BicgVecs<T> &v = w.v;
@@ -1057,7 +1077,7 @@ static ohm_status bicg_start(ohm_backend *b, const DevCsr &a, const PrecondDev &
                      v.r, v.rh, v.p, v.v, o.shadow == OHM_SHADOW_HASHED ? 1 : 0, o.warm ? 1 : 0,
                      o.tol, o.tol_floor, o.tol_mode,
                      (int)std::min<int64_t>(o.max_iters, 0x7fffffff), o.scaled_breakdown ? 1 : 0,
-                     o.forcing, st, pp, stop ? 1 : 0);
+                     o.forcing, st, pp, stop ? 1 : 0, static_cast<uint64_t *>(clear), (int64_t)clear_words);
   b->dispatches += 2;
   return OHM_OK;
 }
@@ -1131,12 +1151,21 @@ static ohm_status bicg_drive(ohm_backend *b, const DevCsr &a, const PrecondDev &
       return fail(OHM_ERR_SOLVE, "Solve error: BiCGSTAB state did not advance (%lld enqueued)",
                   (long long)enqueued);
   }
-  out.status = h->status;
-  out.iters = h->iters;
-  out.r0 = h->r0;
-  out.res = sqrt(h->res2);
-  out.eta = h->eta;
+  bicg_out(h, out);
   OHM_HIP(hipGetLastError());
+  return OHM_OK;
+}
+
+// The backend's workspace for resident solves, at least `bytes` long.
+static ohm_status resident_ws(ohm_backend *b, size_t bytes, void **ws) {
+  if (b->resident_ws_bytes < bytes) {
+    if (b->resident_ws) OHM_HIP(hipFree(b->resident_ws));
+    b->resident_ws = nullptr;
+    b->resident_ws_bytes = 0;
+    OHM_HIP(hipMalloc(&b->resident_ws, bytes));
+    b->resident_ws_bytes = bytes;
+  }
+  *ws = b->resident_ws;
   return OHM_OK;
 }
 
@@ -1146,6 +1175,29 @@ template <typename T>
 static ohm_status bicg_core(ohm_backend *b, const DevCsr &a, const PrecondDev &p, const T *rhs,
                             Workspace<T> &w, const BicgOpts &o, BicgOut &out) {
   Parts pp;
+  const ResGeo geo = resident_geometry(b, a, p, a.n);
+  if (geo.grid && o.check_interval <= 0) {
+    const ResLayout lay = resident_layout(geo, p, a.n, std::is_same<T, float>::value);
+    void *ws = w.resident;
+    if (!ws) OHM_TRY(resident_ws(b, lay.bytes, &ws));
+    if (!w.resident || lay.bytes <= w.resident_bytes) {
+      ResidentGuard guard(true);
+      OHM_TRY(bicg_start<T>(b, a, p, rhs, w, o, pp, nullptr, ws, lay.clear_words));
+      OHM_TRY(resident_enqueue<T>(b, a, p, geo, ws, w.v, w.st));
+      StatusWord *h = reinterpret_cast<StatusWord *>(b->h_pinned);
+      OHM_HIP(hipMemcpyAsync(h, &w.st->status, sizeof(StatusWord), hipMemcpyDeviceToHost,
+                             b->stream));
+      OHM_HIP(hipStreamSynchronize(b->stream));
+      b->readbacks++;
+      out.polls++;
+      if (h->status != ST_RUNNING) {
+        bicg_out(h, out);
+        return OHM_OK;
+      }
+      // given up before any step: the pipeline takes the started solve over
+      return bicg_drive<T>(b, a, p, w, o, pp, false, 0, out);
+    }
+  }
   OHM_TRY(bicg_start<T>(b, a, p, rhs, w, o, pp));
   // The first chunk goes out behind k_init without a poll: the rare solve
   // that k_init ends (b = 0, rho breakdown; under OHM_TOL_INITIAL a warm
@@ -1164,6 +1216,8 @@ static ohm_status bicg_core(ohm_backend *b, const DevCsr &a, const PrecondDev &p
 struct CapturedSolve {
   Workspace<double> w;
   double *vecs = nullptr, *partials = nullptr;
+  void *resident = nullptr;
+  ResGeo geo;
   SolveState *st = nullptr;
   Parts pp{};
   int n = 0;
@@ -1171,13 +1225,15 @@ struct CapturedSolve {
 
 ohm_status captured_create(ohm_backend *b, const DevCsr &a, const PrecondDev &p, double *x,
                            CapturedSolve **out) {
-  (void)b;
   CapturedSolve *c = new CapturedSolve();
   const int n = a.n;
   const size_t stride = ws_stride(n);
   hipError_t e = hipMalloc(&c->vecs, sizeof(double) * stride * kWsVectors);
   if (e == hipSuccess) e = hipMalloc(&c->st, sizeof(SolveState));
   if (e == hipSuccess) e = hipMalloc(&c->partials, sizeof(double) * parts_doubles(a, p, n));
+  c->geo = resident_geometry(b, a, p, n);
+  if (e == hipSuccess && c->geo.grid)
+    e = hipMalloc(&c->resident, resident_layout(c->geo, p, n, false).bytes);
   if (e != hipSuccess) {
     captured_free(c);
     return hip_fail(e, "hipMalloc (captured solve workspace)", __FILE__, __LINE__);
@@ -1197,6 +1253,7 @@ void captured_free(CapturedSolve *c) {
   if (c->vecs) (void)hipFree(c->vecs);
   if (c->st) (void)hipFree(c->st);
   if (c->partials) (void)hipFree(c->partials);
+  if (c->resident) (void)hipFree(c->resident);
   delete c;
 }
 
@@ -1206,6 +1263,12 @@ ohm_status captured_enqueue(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
                             const PrecondDev &p, const double *rhs, const BicgOpts &o, int iters,
                             const int *stop) {
   if (a.n != c->n) return fail(OHM_ERR_INVALID, "captured solve: dimension mismatch");
+  if (c->geo.grid) {
+    // the whole solve in one node; given up, it stays RUNNING and pauses
+    OHM_TRY(bicg_start<double>(b, a, p, rhs, c->w, o, c->pp, stop, c->resident,
+                               resident_layout(c->geo, p, a.n, false).clear_words));
+    return resident_enqueue<double>(b, a, p, c->geo, c->resident, c->w.v, c->st);
+  }
   OHM_TRY(bicg_start<double>(b, a, p, rhs, c->w, o, c->pp, stop));
   for (int k = 0; k < iters; k++) enqueue_any<double>(b, a, p, c->w.v, c->st, c->n, c->pp);
   enqueue_check(b, c->st, c->pp);
@@ -1529,6 +1592,8 @@ ohm_status bicg_solve_f64_noalloc(ohm_backend *b, const DevCsr &a, const Precond
   ws_views(w, (double *)base, stride);
   w.st = (SolveState *)(base + st_off);
   w.partials = (double *)(base + part_off);
+  w.resident = base + align256(need);
+  w.resident_bytes = kScratchBytes - std::min(kScratchBytes, align256(need));
   w.n = n;
   o.eager = true;
   if (o.warm)

@@ -100,6 +100,7 @@ void ohm_backend_destroy(ohm_backend *b) {
   (void)hipStreamSynchronize(b->stream);
   graph_cache_clear(b);
   if (b->d_partials) (void)hipFree(b->d_partials);
+  if (b->resident_ws) (void)hipFree(b->resident_ws);
   if (b->d_counter) (void)hipFree(b->d_counter);
   if (b->d_scalars) (void)hipFree(b->d_scalars);
   if (b->h_pinned) (void)hipHostFree(b->h_pinned);

@@ -114,6 +114,8 @@ struct DevCsr {
   double *t_val = nullptr;         // values of A^T in its CSR order (gathered via t_src)
   int tuned_rows = kSpmvRowsPerBlock, tuned_nnz = kSpmvNnzPerBlock;  // row-block shape
   int per = kSpmvNnzPerBlock / kBlock;  // entries per thread: tuned_nnz / kBlock
+  // rows with more than 4, 6 and 8 entries, of A and of A^T (-1: not counted)
+  int long_rows[3] = {-1, -1, -1}, t_long_rows[3] = {-1, -1, -1};
   std::vector<uint32_t> h_rowptr, h_col; // host copy of the pattern
 };
 
@@ -148,6 +150,8 @@ struct ohm_backend {
   uint64_t ac_ws_gen = 0;            // bumped by every chunk written into ac_ws
   void *dense_ws = nullptr;          // dense LU: n*n matrix + rhs + flag (grow-only)
   size_t dense_ws_bytes = 0;
+  void *resident_ws = nullptr;       // resident solve's workspace (grow-only)
+  size_t resident_ws_bytes = 0;
   void *scratch = nullptr;           // this device's address of the allocation-free
                                      // solve's static scratch array (never freed)
   int64_t dispatches = 0, readbacks = 0;
@@ -176,6 +180,8 @@ namespace ohm {
 void build_spmv_blocks(const uint32_t *rowptr, int n, std::vector<uint32_t> &blocks,
                        int rows_cap = kSpmvRowsPerBlock, int nnz_cap = kSpmvNnzPerBlock);
 int spmv_default_per(const uint32_t *rowptr, int n);
+// Rows with more than 4, 6 and 8 entries.
+void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]);
 // Pick the fastest (rows_cap, nnz_cap) for m by timing each candidate.
 // fused: m is applied by the fused BiCGSTAB kernels (keep 256-row blocks)
 ohm_status csr_autotune(ohm_backend *b, DevCsr &m, int *rows_out, int *nnz_out,

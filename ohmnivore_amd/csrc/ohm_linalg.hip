@@ -63,6 +63,16 @@ int spmv_default_per(const uint32_t *rowptr, int n) {
   return spmv_per_for(std::max(mean, 1) * kBlock);
 }
 
+void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]) {
+  out[0] = out[1] = out[2] = 0;
+  for (int r = 0; r < n; r++) {
+    const uint32_t c = rowptr[r + 1] - rowptr[r];
+    out[0] += c > 4;
+    out[1] += c > 6;
+    out[2] += c > 8;
+  }
+}
+
 // Device block table: (first row, first nonzero) of every block boundary, so
 // a workgroup reads its row and nonzero ranges with one 16-byte scalar load.
 std::vector<uint32_t> spmv_block_pairs(const uint32_t *rowptr, const std::vector<uint32_t> &bounds) {
@@ -271,6 +281,7 @@ ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32
   m.nnz = nnz;
   m.h_rowptr.assign(rowptr, rowptr + n + 1);
   m.h_col.assign(col, col + nnz);
+  count_long_rows(rowptr, n, m.long_rows);
   std::vector<uint32_t> bounds;
   m.per = spmv_default_per(rowptr, n);
   m.tuned_nnz = m.per * kBlock;
@@ -319,6 +330,7 @@ ohm_status csr_ensure_transpose(ohm_backend *b, DevCsr &m) {
       tsrc[p] = (uint32_t)k;
     }
   std::vector<uint32_t> bounds;
+  count_long_rows(trp.data(), n, m.t_long_rows);
   build_spmv_blocks(trp.data(), n, bounds);
   m.t_n_blocks = (int)bounds.size() - 1;
   const std::vector<uint32_t> blocks = spmv_block_pairs(trp.data(), bounds);
@@ -357,6 +369,7 @@ ohm_status csr_transpose_view(ohm_backend *b, DevCsr &m, DevCsr &view) {
   view.val = m.t_val;
   view.blocks = m.t_blocks;
   view.n_blocks = m.t_n_blocks;
+  std::copy(m.t_long_rows, m.t_long_rows + 3, view.long_rows);
   return OHM_OK;
 }
 

@@ -1,0 +1,57 @@
+// ohm_persist.h — the resident BiCGSTAB solve (ohm_persist.hip): one launch
+// iterates to the end, workgroups meeting through tagged words in memory.
+#pragma once
+
+#include "ohm_precond.h"
+#include "ohm_reduce.h"
+
+namespace ohm {
+
+constexpr int kResThreads = 512;      // most threads of a workgroup (256 registers each)
+constexpr int kResMaxGrid = 256;      // most workgroups (one per CU)
+constexpr int kResMaxLong = 32;       // rows per matrix beyond the row tile
+constexpr int kResSlotWords = 8;      // 64-bit words of one reduction slot
+
+// How a solve is cut: `grid` workgroups of `threads` threads with `rows`
+// consecutive rows each, one per thread, row tiles of `width` entries.
+// grid == 0: the system does not fit this path.
+struct ResGeo {
+  int grid = 0, threads = 0, rows = 0, width = 0;
+};
+// The geometry of a solve of a x = b with p.
+ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n);
+
+// Workspace of one solve, cleared before it: tagged vectors, reduction slots
+// and the outcome word.
+struct ResLayout {
+  size_t clear_words = 0, bytes = 0;  // the whole workspace
+  size_t slots = 0, outcome = 0;      // word offsets
+};
+ResLayout resident_layout(const ResGeo &g, const PrecondDev &p, int n, bool f32);
+
+// Enqueues the solve behind k_init: x, r and r_hat as k_init left them, the
+// workspace `ws` with its first clear_words words zero. On success the state
+// word holds the final status; a solve that could not finish (its workgroups
+// did not all run at once within the time limit) leaves every vector and the
+// state as k_init did, RUNNING, for the multi-kernel pipeline.
+template <typename T>
+ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p, const ResGeo &g,
+                            void *ws, const BicgVecs<T> &v, SolveState *st);
+
+// One resident solve at a time per process: two that share the GPU could each
+// hold the compute units the other waits for.
+void resident_lock();
+void resident_unlock();
+struct ResidentGuard {
+  bool on;
+  explicit ResidentGuard(bool take) : on(take) {
+    if (on) resident_lock();
+  }
+  ~ResidentGuard() {
+    if (on) resident_unlock();
+  }
+  ResidentGuard(const ResidentGuard &) = delete;
+  ResidentGuard &operator=(const ResidentGuard &) = delete;
+};
+
+}  // namespace ohm

@@ -1,0 +1,115 @@
+"""The resident BiCGSTAB solve (one launch for the whole solve, workgroups of
+at most 512 rows meeting through memory) against the FP64 LU and against the
+multi-kernel pipeline, which a check_interval of one's own selects, at the
+edges of its dispatch: one workgroup and several, a last workgroup of few
+rows, row tiles of 4, 6 and 8 entries, rows longer than a tile, no
+preconditioner, FP32 refinement, warm starts and breakdowns."""
+import numpy as np
+import pytest
+
+import oracle
+from ohmnivore_amd import _native as N
+from ohmnivore_amd import solver
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def be():
+    return solver.HipBackend()
+
+
+def system(n, per_row, n_dense, seed):
+    """Diagonally dominant, about per_row entries a row (neighbours and far
+    columns), the first n_dense rows coupled to every third unknown."""
+    rng = np.random.default_rng(seed)
+    rows, cols, vals = [], [], []
+    for d in range(1, (per_row - 1) // 2 + 1):
+        step = 1 if d == 1 else max(2, n // (d + 1))
+        i = np.arange(n - step) if n > step else np.arange(0)
+        for r, c in ((i, i + step), (i + step, i)):
+            rows.append(r)
+            cols.append(c)
+            vals.append(-rng.uniform(0.1, 1.0, r.shape[0]))
+    for k in range(n_dense):
+        c = np.arange(k + 1, n, 3)
+        rows.append(np.full(c.shape[0], k))
+        cols.append(c)
+        vals.append(-rng.uniform(0.0, 0.01, c.shape[0]))
+    rows, cols, vals = (np.concatenate(v) for v in (rows, cols, vals))
+    diag = np.ones(n)
+    np.add.at(diag, rows, np.abs(vals))
+    return oracle.from_triplet_arrays(n, n, np.concatenate([rows, np.arange(n)]),
+                                      np.concatenate([cols, np.arange(n)]),
+                                      np.concatenate([vals, 2.0 * diag]))
+
+
+def solve(be, a, b, prec, x0=None, **kw):
+    m = be.upload_matrix(a.values, a.col_indices, a.row_pointers, a.nrows)
+    p = None if prec == N.PREC_NONE else be.preconditioner(m, prec)
+    bb, xx = be.new_buffer(a.nrows), be.new_buffer(a.nrows)
+    be.upload_vec(b, bb)
+    if x0 is not None:
+        be.upload_vec(x0, xx)
+    st = be.bicgstab(m, bb, xx, p, solver.bicgstab_params(warm_start=x0 is not None, **kw))
+    return be.download_vec(xx), st
+
+
+# relative residual 1e-13 and a condition number below 10: errors below 1e-11
+TOL = dict(tolerance=1e-13, max_iterations=2000)
+
+
+@pytest.mark.parametrize("n", [65, 511, 512, 513, 1024, 1025, 5000])
+@pytest.mark.parametrize("per_row,n_dense", [(3, 0), (5, 1), (7, 2)])
+@pytest.mark.parametrize("prec", [N.PREC_NONE, N.PREC_JACOBI, N.PREC_ISAI],
+                         ids=["none", "jacobi", "isai"])
+def test_resident_matches_lu_and_pipeline(be, n, per_row, n_dense, prec):
+    a = system(n, per_row, n_dense, seed=n + per_row)
+    b = np.random.default_rng(n).standard_normal(n)
+    ref = oracle.sparse_lu_solve(a, b)
+    scale = np.abs(ref).max()
+    x, st = solve(be, a, b, prec, **TOL)
+    y, _ = solve(be, a, b, prec, check_interval=8, **TOL)
+    assert st.iterations > 0 and st.residual_norm < 1e-12
+    assert np.abs(x - ref).max() < 1e-11 * scale
+    assert np.abs(y - ref).max() < 1e-11 * scale
+    # the answer does not depend on when workgroups meet
+    assert solve(be, a, b, prec, **TOL)[0].tobytes() == x.tobytes()
+
+
+@pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_ISAI], ids=["jacobi", "isai"])
+def test_resident_is_one_launch_per_solve(be, prec):
+    a = system(3000, 5, 0, seed=5)
+    b = np.ones(3000)
+    _, st = solve(be, a, b, prec, **TOL)
+    _, pl = solve(be, a, b, prec, check_interval=8, **TOL)
+    assert st.dispatches < 8 < pl.dispatches
+
+
+@pytest.mark.parametrize("n", [300, 1600])
+@pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_ISAI], ids=["jacobi", "isai"])
+def test_resident_fp32_refinement_and_warm_start(be, n, prec):
+    a = system(n, 5, 1, seed=n)
+    b = np.random.default_rng(n).standard_normal(n)
+    ref = oracle.sparse_lu_solve(a, b)
+    x, _ = solve(be, a, b, prec, precision="fp32_ir", tolerance=1e-12, max_iterations=2000)
+    assert np.abs(x - ref).max() < 1e-10 * np.abs(ref).max()
+    y, st = solve(be, a, b, prec, x0=ref + 1e-6, **TOL)
+    assert np.abs(y - ref).max() < 1e-11 * np.abs(ref).max()
+    z, st0 = solve(be, a, b, prec, x0=y, tolerance=1e-9)
+    assert st0.iterations == 0 and z.tobytes() == y.tobytes()
+    assert st.iterations > 0
+
+
+def test_resident_stops(be):
+    """The iteration cap, a zero right-hand side and an unreachable one end as
+    in the pipeline."""
+    a = system(700, 5, 0, seed=1)
+    b = np.ones(700)
+    for kw in (dict(check_interval=8), {}):
+        with pytest.raises(N.OhmnivoreError, match="did not converge within 2 iterations"):
+            solve(be, a, b, N.PREC_JACOBI, tolerance=1e-14, max_iterations=2, **kw)
+        with pytest.raises(N.OhmnivoreError, match="NaN/Inf|breakdown"):
+            solve(be, a, np.where(np.arange(700) == 690, np.inf, b), N.PREC_JACOBI, **kw)
+    x, st = solve(be, a, np.zeros(700), N.PREC_JACOBI)
+    assert not x.any() and st.iterations == 0
