@@ -829,7 +829,7 @@ ohm_status ohm_newton_run(ohm_newton_ctx *c, const ohm_newton_params *params,
   for (it = 0; it < prm.max_iterations; it++) {
     hipLaunchKernelGGL(k_copy_d, dim3(grid_for(n, 4)), dim3(kBlock), 0, st, n, c->x, c->x_old);
     enqueue_eval_assemble(c, c->x);
-    OHM_TRY(precond_refresh(b, c->A, c->P));
+    if (prm.linear_solver != OHM_LINEAR_DENSE_LU) OHM_TRY(precond_refresh(b, c->A, c->P));
     o.tol = prm.bicgstab_tolerance;
     o.forcing = fc;
     BicgOut bo;
