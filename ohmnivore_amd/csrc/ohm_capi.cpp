@@ -79,7 +79,7 @@ ohm_status ohm_backend_create(int device, ohm_backend **out) {
   OHM_HIP(hipMalloc(&b->d_counter, sizeof(unsigned) * 4));
   OHM_HIP(hipMemset(b->d_counter, 0, sizeof(unsigned) * 4));
   OHM_HIP(hipMalloc(&b->d_scalars, sizeof(double) * 16));
-  OHM_HIP(hipHostMalloc((void **)&b->h_pinned, sizeof(double) * 16, hipHostMallocDefault));
+  OHM_HIP(hipHostMalloc((void **)&b->h_pinned, kPinnedBytes, hipHostMallocDefault));
   OHM_HIP(hipEventCreate(&b->ev0));
   OHM_HIP(hipEventCreate(&b->ev1));
   ohm_status s = ensure_partials(b, (size_t)kMaxReduceBlocks * 4);

@@ -63,6 +63,7 @@ inline void with_per(int per, F &&f) {
     default: f(std::integral_constant<int, 8>()); break;
   }
 }
+constexpr size_t kPinnedBytes = 512;     // host staging of status words
 constexpr int64_t kDeferMaxReads = int64_t(1) << 21;  // consumer x producer workgroups re-summed
 
 // ----------------------------------------------------------- solve state --

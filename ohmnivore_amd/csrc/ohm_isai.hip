@@ -28,7 +28,7 @@
 #include <cmath>
 #include <unordered_map>
 
-#include "ohm_precond.h"
+#include "ohm_isai_dev.h"
 #include "ohm_spmv.h"
 
 namespace ohm {
@@ -107,15 +107,7 @@ __global__ void k_ilu_init(int64_t nf, const int32_t *__restrict__ from_a,
                            double *__restrict__ f) {
   for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < nf;
        e += (int64_t)gridDim.x * kBlock) {
-    int32_t s = from_a[e];
-    double v = s >= 0 ? aval[s] : 0.0;
-    int32_t d = div[e];
-    if (d >= 0) {
-      int32_t ad = from_a[d];
-      double piv = ad >= 0 ? aval[ad] : 0.0;
-      v = fabs(piv) < 1e-30 ? 0.0 : v / piv;
-    }
-    f[e] = v;
+    f[e] = ilu_start(e, from_a, div, aval);
   }
 }
 
@@ -125,15 +117,7 @@ __global__ void k_ilu_sweep(int64_t nf, const int32_t *__restrict__ from_a,
                             const double *__restrict__ fin, double *__restrict__ fout) {
   for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < nf;
        e += (int64_t)gridDim.x * kBlock) {
-    int32_t s = from_a[e];
-    double v = s >= 0 ? aval[s] : 0.0;
-    for (uint32_t q = ptr[e]; q < ptr[e + 1]; q++) v -= fin[pairs[2 * q]] * fin[pairs[2 * q + 1]];
-    int32_t d = div[e];
-    if (d >= 0) {
-      double piv = fin[d];
-      v = fabs(piv) < 1e-30 ? 0.0 : v / piv;
-    }
-    fout[e] = v;
+    fout[e] = ilu_entry(e, from_a, div, ptr, pairs, aval, fin);
   }
 }
 
@@ -145,14 +129,7 @@ __global__ void k_isai_sweep(int64_t m, const uint32_t *__restrict__ ptr,
                              const double *__restrict__ min, double *__restrict__ mout) {
   for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < m;
        e += (int64_t)gridDim.x * kBlock) {
-    double v = is_k[e] ? 1.0 : 0.0;
-    for (uint32_t q = ptr[e]; q < ptr[e + 1]; q++) v -= f[dep[2 * q]] * min[dep[2 * q + 1]];
-    int32_t d = diag[e];
-    if (d >= 0) {
-      double piv = f[d];
-      v = fabs(piv) < 1e-30 ? 0.0 : v / piv;
-    }
-    mout[e] = v;
+    mout[e] = isai_entry(e, ptr, dep, diag, is_k, f, min);
   }
 }
 
@@ -174,17 +151,8 @@ __global__ __launch_bounds__(kSweepWg) void k_ilu_sweeps_wg(
     const double *__restrict__ aval, double *f0, double *f1, int sweeps) {
   double *fin = f0, *fout = f1;
   for (int s = 0; s < sweeps; s++) {
-    for (int64_t e = threadIdx.x; e < nf; e += kSweepWg) {
-      int32_t src = from_a[e];
-      double v = src >= 0 ? aval[src] : 0.0;
-      for (uint32_t q = ptr[e]; q < ptr[e + 1]; q++) v -= fin[pairs[2 * q]] * fin[pairs[2 * q + 1]];
-      int32_t d = div[e];
-      if (d >= 0) {
-        double piv = fin[d];
-        v = fabs(piv) < 1e-30 ? 0.0 : v / piv;
-      }
-      fout[e] = v;
-    }
+    for (int64_t e = threadIdx.x; e < nf; e += kSweepWg)
+      fout[e] = ilu_entry(e, from_a, div, ptr, pairs, aval, fin);
     __syncthreads();
     double *t = fin;
     fin = fout;
@@ -198,16 +166,8 @@ __global__ __launch_bounds__(kSweepWg) void k_isai_sweeps_wg(
     const double *__restrict__ f, double *m0, double *m1, int sweeps) {
   double *min = m0, *mout = m1;
   for (int s = 0; s < sweeps; s++) {
-    for (int64_t e = threadIdx.x; e < m; e += kSweepWg) {
-      double v = is_k[e] ? 1.0 : 0.0;
-      for (uint32_t q = ptr[e]; q < ptr[e + 1]; q++) v -= f[dep[2 * q]] * min[dep[2 * q + 1]];
-      int32_t d = diag[e];
-      if (d >= 0) {
-        double piv = f[d];
-        v = fabs(piv) < 1e-30 ? 0.0 : v / piv;
-      }
-      mout[e] = v;
-    }
+    for (int64_t e = threadIdx.x; e < m; e += kSweepWg)
+      mout[e] = isai_entry(e, ptr, dep, diag, is_k, f, min);
     __syncthreads();
     double *t = min;
     min = mout;
@@ -693,6 +653,31 @@ void precond_apply_f32(ohm_backend *b, const PrecondDev &p, const float *in, flo
                        out, st, skip);
     b->dispatches++;
   }
+}
+
+bool isai_view(const PrecondDev &p, IsaiView &v) {
+  const IsaiPlan *pl = p.plan;
+  if (!pl || p.mm.rowptr || pl->nnz_f > kSweepWgMax) return false;
+  v.nf = pl->nnz_f;
+  v.from_a = pl->f_from_a;
+  v.div = pl->f_div;
+  v.cp_ptr = pl->cp_ptr;
+  v.cp_pairs = pl->cp_pairs;
+  v.f0 = pl->f_val;
+  v.f1 = pl->f_tmp;
+  v.ilu_sweeps = p.ilu_sweeps;
+  for (int k = 0; k < 2; k++) {
+    const IsaiPlan::Side &s = pl->side[k];
+    const DevCsr &m = k == 0 ? p.ml : p.mu;
+    if (s.m > kSweepWgMax) return false;
+    v.side[k] = {s.m, s.dep_ptr, s.dep, s.diag, s.is_k, s.out_pos, s.m0, s.m1, s.sweeps, m.val,
+                 p.has_f32 ? m.val32 : nullptr};
+  }
+  return true;
+}
+
+void isai_started(PrecondDev &p) {
+  if (p.plan) p.plan->f_init = true;
 }
 
 void isai_reset(PrecondDev &p) {

@@ -26,6 +26,8 @@ ohm_status precond_ensure_f32(ohm_backend *b, PrecondDev &p);
 void precond_free(PrecondDev &p);
 // forget the ILU(0) factors so the next refresh restarts from A
 void isai_reset(PrecondDev &p);
+// the ILU(0) factors in the plan come from a refresh done elsewhere
+void isai_started(PrecondDev &p);
 // out = M^-1 in (f64), skipping per the solve state like the SpMV kernels
 void precond_apply(ohm_backend *b, const PrecondDev &p, const double *in, double *out, double *tmp,
                    const SolveState *st, int skip);
@@ -130,6 +132,8 @@ ohm_status captured_enqueue(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
 ohm_status captured_resume(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
                            const PrecondDev &p, const BicgOpts &o, int64_t enqueued,
                            BicgOut &out);
+// Whether a system of n unknowns takes the one-wave solve.
+bool fused_small(int n);
 ohm_status status_to_error(int status, int64_t iters, int64_t max_iters);
 
 }  // namespace ohm

@@ -116,6 +116,42 @@ __device__ __forceinline__ void spmv_block(const uint32_t *__restrict__ rowptr,
       [] { return true; }, [](const Opnd<T, 1> &o) { return o.v[0]; }, f);
 }
 
+// inv[r] = 1/a_rr when |a_rr| > 1e-30 (src/solver/gpu.rs:178-189). For a
+// zero-diagonal row (V-source / inductor branch) inv[r] = 1/S_rr with
+// S_rr = -sum_j a_rj a_jr / a_jj the diagonal of the Schur complement over
+// the rows that do have a pivot; 1 when that sum is zero too.
+__device__ __forceinline__ void jacobi_row(int r, const uint32_t *__restrict__ rowptr,
+                                           const uint32_t *__restrict__ col,
+                                           const double *__restrict__ val,
+                                           const int32_t *__restrict__ diag_pos, double *inv,
+                                           float *inv32) {
+  int dp = diag_pos[r];
+  double d = dp >= 0 ? val[dp] : 0.0;
+  double out;
+  if (fabs(d) > 1e-30) {
+    out = 1.0 / d;
+  } else {
+    double s = 0.0;
+    for (uint32_t k = rowptr[r]; k < rowptr[r + 1]; k++) {
+      uint32_t j = col[k];
+      if ((int)j == r) continue;
+      int dj = diag_pos[j];
+      double ajj = dj >= 0 ? val[dj] : 0.0;
+      if (fabs(ajj) <= 1e-30) continue;
+      double ajr = 0.0;  // a_jr: search row j
+      for (uint32_t q = rowptr[j]; q < rowptr[j + 1]; q++)
+        if ((int)col[q] == r) {
+          ajr = val[q];
+          break;
+        }
+      s -= val[k] * ajr / ajj;
+    }
+    out = (fabs(s) > 1e-300) ? 1.0 / s : 1.0;
+  }
+  inv[r] = out;
+  if (inv32) inv32[r] = (float)out;
+}
+
 __device__ __forceinline__ bool solve_stopped(const SolveState *st, int skip) {
   if (!st || !skip) return false;
   return st->status != ST_RUNNING || (skip == 2 && st->s_conv);
