@@ -36,152 +36,12 @@
 #include <tuple>
 #include <vector>
 
+#include "ohm_batch_resident.h"
 #include "ohm_persist.h"
 #include "ohm_reduce.h"
 #include "ohm_sources.h"
 
 namespace ohm {
-
-// ------------------------------------------------------------ scalars ----
-template <typename R>
-struct cx {
-  R re, im;
-};
-template <typename R>
-__device__ __forceinline__ cx<R> operator+(cx<R> a, cx<R> b) {
-  return {a.re + b.re, a.im + b.im};
-}
-template <typename R>
-__device__ __forceinline__ cx<R> operator-(cx<R> a, cx<R> b) {
-  return {a.re - b.re, a.im - b.im};
-}
-template <typename R>
-__device__ __forceinline__ cx<R> operator*(cx<R> a, cx<R> b) {
-  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-
-template <typename S>
-struct Tr;
-template <>
-struct Tr<double> {
-  using R = double;
-  static constexpr bool C = false;
-};
-template <>
-struct Tr<float> {
-  using R = float;
-  static constexpr bool C = false;
-};
-template <>
-struct Tr<cx<double>> {
-  using R = double;
-  static constexpr bool C = true;
-};
-template <>
-struct Tr<cx<float>> {
-  using R = float;
-  static constexpr bool C = true;
-};
-
-template <typename S>
-__device__ __forceinline__ S mk(double re, double im) {
-  using R = typename Tr<S>::R;
-  if constexpr (Tr<S>::C)
-    return S{(R)re, (R)im};
-  else
-    return (S)re;
-}
-template <typename S>
-__device__ __forceinline__ S zero() {
-  return mk<S>(0.0, 0.0);
-}
-template <typename S>
-__device__ __forceinline__ double re_of(S a) {
-  if constexpr (Tr<S>::C)
-    return (double)a.re;
-  else
-    return (double)a;
-}
-template <typename S>
-__device__ __forceinline__ double im_of(S a) {
-  if constexpr (Tr<S>::C)
-    return (double)a.im;
-  else
-    return 0.0;
-}
-
-// a_k = g_k + sigma c_k on the fly
-template <typename S>
-__device__ __forceinline__ S aval(typename Tr<S>::R g, typename Tr<S>::R c, double sr, double si) {
-  using R = typename Tr<S>::R;
-  if constexpr (Tr<S>::C)
-    return S{g + (R)sr * c, (R)si * c};
-  else
-    return g + (R)sr * c;
-}
-
-// conj(a) . b and ||a||^2 accumulators (compensated in FP32)
-template <typename S>
-struct DotAcc {
-  Acc<typename Tr<S>::R> re, im;
-  __device__ __forceinline__ void add(S a, S b) {
-    if constexpr (Tr<S>::C) {
-      re.add_prod(a.re, b.re);
-      re.add_prod(a.im, b.im);
-      im.add_prod(a.re, b.im);
-      im.add_prod(-a.im, b.re);
-    } else {
-      re.add_prod(a, b);
-    }
-  }
-};
-template <typename S>
-struct NrmAcc {
-  Acc<typename Tr<S>::R> s;
-  __device__ __forceinline__ void add(S a) {
-    if constexpr (Tr<S>::C) {
-      s.add_prod(a.re, a.re);
-      s.add_prod(a.im, a.im);
-    } else {
-      s.add_prod(a, a);
-    }
-  }
-};
-
-// double-precision complex helpers for the per-system scalar algebra
-struct zd {
-  double re, im;
-};
-__device__ __forceinline__ zd zmul(zd a, zd b) {
-  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-__device__ __forceinline__ zd zdiv(zd a, zd b) {
-  const double d = b.re * b.re + b.im * b.im;
-  return {(a.re * b.re + a.im * b.im) / d, (a.im * b.re - a.re * b.im) / d};
-}
-__device__ __forceinline__ double zabs2(zd a) { return a.re * a.re + a.im * a.im; }
-
-// ---------------------------------------------------------- batch state --
-struct BSys {
-  double rho[2], alpha[2], omega[2], beta[2];
-  double abs_tol, bnorm2, rr, ss, rhrh;
-  int status, s_conv, iters, max_iters;
-  unsigned counter;
-  int scaled;
-  int started;  // persistent kernel: scalars below the vectors are live
-  int pad;
-};
-
-struct BGeo {
-  const uint32_t *rowptr, *col;
-  const double *g, *c;      // c may be null (then sigma is ignored)
-  const float *g32, *c32;
-  double sig_re, sig_im;
-  int64_t off;              // offset of this system in the concatenated vectors
-  int n;
-  int first_block, n_blocks;
-  int pad;
-};
 
 struct BBlock {
   int sys;
@@ -191,28 +51,6 @@ struct BBlock {
 
 constexpr int kPersistRows = 4096;  // systems this small run in the persistent kernel
 constexpr int kBatchPartials = 5;   // most partial sums one reduction writes
-
-template <typename S>
-__device__ __forceinline__ const typename Tr<S>::R *gvals(const BGeo &q) {
-  if constexpr (sizeof(typename Tr<S>::R) == 8)
-    return q.g;
-  else
-    return q.g32;
-}
-template <typename S>
-__device__ __forceinline__ const typename Tr<S>::R *cvals(const BGeo &q) {
-  if constexpr (sizeof(typename Tr<S>::R) == 8)
-    return q.c;
-  else
-    return q.c32;
-}
-
-template <typename S>
-__device__ __forceinline__ S load_a(const BGeo &q, const typename Tr<S>::R *g,
-                                    const typename Tr<S>::R *c, uint32_t k) {
-  using R = typename Tr<S>::R;
-  return aval<S>(g[k], c ? c[k] : (R)0, q.sig_re, q.sig_im);
-}
 
 // Sum K values over the workgroup for one system; the last block of the
 // system (ticket on its BSys) returns true with the system totals in
@@ -314,10 +152,6 @@ __device__ __forceinline__ void bspmv_block(const BGeo &q, const BBlock &bk,
   }
 }
 
-__device__ __forceinline__ bool brk_small(double num_abs, double scale, int scaled,
-                                          double abs_thresh) {
-  return scaled ? num_abs <= 1e-30 * scale : num_abs < abs_thresh;
-}
 
 // --------------------------------------------------------------- kernels --
 __global__ void k_bsys_reset(int K, BSys *sys, const int *__restrict__ active, int max_iters,
@@ -1025,6 +859,7 @@ struct ohm_batch {
   double *d_scale = nullptr;
   std::vector<void *> allocs;    // patterns and values
   std::vector<int64_t> h_nnz;    // per system
+  std::vector<int> h_long;       // per system: rows with more than 4, 6 and 8 entries
   bool has_f32 = false;
   bool jac64_valid = false, jac32_valid = false;  // Jacobi inverses match the current sigmas
   // workspaces: 10 vectors each (x r rh p v s t ph sh inv) + rhs/ax scratch
@@ -1125,6 +960,18 @@ void enqueue_iter(ohm_batch *bt, BW<S> &w, int nblk) {
   bt->owner->dispatches += 9;
 }
 
+// r, r_hat and the scalars of every running system's start.
+template <typename S>
+void enqueue_start(ohm_batch *bt, BW<S> &w, int nblk, const BInitArgs &ia) {
+  hipStream_t st = bt->owner->stream;
+  hipLaunchKernelGGL(k_binit<S>, dim3(nblk), dim3(kBlock), 0, st, bt->d_active, bt->d_geo,
+                     bt->d_sys, w.b, w.ax, w.x, w.r, w.rh, w.p, w.v, ia, bt->d_partials);
+  hipLaunchKernelGGL(k_bfold_init<S>, dim3(bt->K), dim3(kBlock), 0, st, bt->d_geo, bt->d_sys, ia,
+                     bt->d_partials);
+  bt->dispatches += 2;
+  bt->owner->dispatches += 2;
+}
+
 struct BatchOpts {
   int64_t max_iters = 10000;
   double tol = 1e-5;
@@ -1178,6 +1025,30 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
   bt->dispatches += 3;
   b->dispatches += 3;
 
+  // resident path: every running system's workgroups on the chip at once. A
+  // system that comes back RUNNING (given up) is solved below.
+  if constexpr (sizeof(typename Tr<S>::R) == 8) {
+    std::vector<BatchSolve<S>> list;
+    for (int k = 0; k < K; k++)
+      if (run[k] && bt->h_geo[k].n > 0) {
+        const int64_t off = bt->h_geo[k].off;
+        list.push_back({&bt->h_geo[k], &bt->h_long[3 * (size_t)k], w.x + off, w.r + off, w.rh + off,
+                        pk == PK_JACOBI ? w.inv + off : nullptr, bt->d_sys + k});
+      }
+    if (o.check_interval <= 0 && batch_resident_fits<S>(b, list)) {
+      ResidentGuard guard(true);
+      enqueue_start<S>(bt, w, (int)tab.size(), ia);
+      OHM_TRY(batch_resident_enqueue<S>(b, list));
+      OHM_HIP(hipMemcpyAsync(bt->h_sys, bt->d_sys, sizeof(BSys) * K, hipMemcpyDeviceToHost,
+                             stream));
+      OHM_HIP(hipStreamSynchronize(stream));
+      b->readbacks++;
+      bool all = true;
+      for (int k = 0; k < K; k++) all = all && !(run[k] && bt->h_sys[k].status == ST_RUNNING);
+      if (all) return OHM_OK;
+    }
+  }
+
   // persistent path: every running system small
   int max_n = 0;
   for (int k = 0; k < K; k++)
@@ -1215,13 +1086,7 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
     return OHM_OK;
   }
 
-  hipLaunchKernelGGL(k_binit<S>, dim3(tab.size()), dim3(kBlock), 0, stream, bt->d_active,
-                     bt->d_geo, bt->d_sys, w.b, w.ax, w.x, w.r, w.rh, w.p, w.v, ia,
-                     bt->d_partials);
-  hipLaunchKernelGGL(k_bfold_init<S>, dim3(K), dim3(kBlock), 0, stream, bt->d_geo, bt->d_sys, ia,
-                     bt->d_partials);
-  bt->dispatches += 2;
-  b->dispatches += 2;
+  enqueue_start<S>(bt, w, (int)tab.size(), ia);
   std::vector<char> live = run;
   int64_t done = 0;
   for (bool first = true;; first = false) {
@@ -1654,6 +1519,9 @@ ohm_status ohm_batch_create(ohm_backend *b, int32_t is_complex, int64_t k,
     g.n_blocks = (int)bt->h_blocks.size() - g.first_block;
     bt->h_geo.push_back(g);
     bt->h_nnz.push_back(nnz);
+    int lr[3] = {0, 0, 0};
+    if (n > 0) count_long_rows(q.rowptr, n, lr);
+    bt->h_long.insert(bt->h_long.end(), lr, lr + 3);
     host_rowptr.push_back(q.rowptr);
     bt->max_n = std::max(bt->max_n, n);
     off += n;

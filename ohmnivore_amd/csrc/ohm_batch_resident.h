@@ -1,0 +1,32 @@
+// ohm_batch_resident.h — resident solves of a batch (ohm_batch_resident.hip).
+#pragma once
+
+#include <vector>
+
+#include "ohm_batch_types.h"
+
+namespace ohm {
+
+// One system of a batch as the resident solve needs it; vectors as k_binit
+// and k_bfold_init left them.
+template <typename S>
+struct BatchSolve {
+  const BGeo *geo;
+  const int *long_rows;   // rows with more than 4, 6 and 8 entries
+  S *x;
+  const S *r, *rh, *inv;  // inv null: no preconditioner
+  BSys *st;
+};
+
+// Whether these systems take the resident path: their workgroups run at once
+// in at most kResBatchGroups launches.
+template <typename S>
+bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys);
+
+// Enqueues the solves. A system that could not finish stays RUNNING with its
+// vectors untouched. The caller holds the resident lock until the launches
+// are done.
+template <typename S>
+ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys);
+
+}  // namespace ohm

@@ -1,0 +1,189 @@
+// ohm_batch_resident.hip — the batch engine's solves as resident launches.
+//
+// A batched iteration is nine launches (five kernels and a fold per reduction,
+// 30 us at 8 systems of 16,388 rows), and a batch of small systems runs one
+// workgroup each with every vector in memory: 21 complex systems of 1,847
+// rows took 35 us per iteration on 21 of 256 compute units. Here each
+// system has its own workgroups, which keep its rows in registers and meet
+// through tagged words as a single resident solve's do (ohm_persist.hip); the
+// systems do not wait for each other. Jacobi or no preconditioner, 64-bit,
+// real or complex (A = G + sigma C formed as the rows are loaded).
+//
+// Bound, as there, by the latency of its reductions and by registers (complex
+// tiles of six entries spill). Systems that do not fit the chip together go in
+// groups, one launch after another; with more than kResBatchGroups of them the
+// nine launches, or a workgroup per system, do as well. Measured, ten
+// backward-Euler steps of 8 x 16,388 real rows 41.8 -> 17.8 ms (1,150
+// iterations); 21 x 1,847 complex rows 16.6 -> 7.3 ms (375 to 481 iterations).
+#include <algorithm>
+
+#include "ohm_batch_resident.h"
+#include "ohm_resident_dev.h"
+
+namespace ohm {
+
+// Rows of a workgroup. Real systems: ten waves leave 168 registers a thread,
+// enough without requests ahead of a reduction. Complex: eight waves, 256.
+template <typename S>
+constexpr int kResBatchRows = Tr<S>::C ? 512 : 640;
+constexpr int kResBatchGroups = 2;
+
+template <typename S, int W>
+__global__ __launch_bounds__(kResBatchRows<S>) void k_batch_resident(
+    const ResArgs<S, BSys> *__restrict__ args, const int *__restrict__ owner, int first) {
+  using R = Resident<S, BSys, PK_JACOBI, W, false>;
+  __shared__ typename R::Shared sh;
+  __shared__ ResArgs<S, BSys> a;
+  extern __shared__ __align__(16) unsigned char res_lds[];
+  if (threadIdx.x == 0) {
+    a = args[owner[first + blockIdx.x]];
+    a.first -= first;  // within this launch
+  }
+  __syncthreads();
+  R r(a, sh, res_lds);
+  r.solve();
+}
+
+__global__ void k_clear_words(int64_t n, u64 *w) {
+  for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kBlock)
+    w[i] = 0;
+}
+
+namespace {
+
+struct Cut {
+  int rows = 0, width = 0;
+  std::vector<int> group;  // first system of each launch, then the number of systems
+};
+
+// Rows per workgroup, tile width and launches of a list of systems; rows == 0
+// when it does not fit.
+template <typename S>
+Cut cut_batch(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
+  Cut c;
+  static const int kWidths[3] = {4, 6, 8}, kLong[3] = {2, 2, kResMaxLong};
+  for (int w = 0; w < 3 && !c.width; w++) {
+    bool fits = true;
+    for (const auto &s : sys) fits = fits && s.long_rows[w] <= kLong[w];
+    if (fits) c.width = kWidths[w];
+  }
+  if (!c.width) return c;
+  const int cus = std::min(b->num_cu, kResMaxGrid);
+  // the smallest workgroups that need the fewest launches; systems of one
+  // workgroup each wait for nobody, so any number of them shares a launch
+  for (int rows : {256, 320, 384, 448, 512, 576, 640}) {
+    if (rows > kResBatchRows<S>) break;
+    std::vector<int> group(1, 0);
+    int used = 0;
+    bool fits = true, waits = false;
+    for (const auto &s : sys) waits = waits || s.geo->n > rows;
+    for (size_t k = 0; waits && k < sys.size(); k++) {
+      const int wgs = (sys[k].geo->n + rows - 1) / rows;
+      fits = fits && wgs <= cus;
+      if (used > 0 && used + wgs > cus) {
+        group.push_back((int)k);
+        used = 0;
+      }
+      used += wgs;
+    }
+    group.push_back((int)sys.size());
+    if (fits && (c.rows == 0 || group.size() < c.group.size())) {
+      c.rows = rows;
+      c.group = group;
+    }
+  }
+  if (c.rows && (int)c.group.size() - 1 > kResBatchGroups) c.rows = 0;
+  return c;
+}
+
+}  // namespace
+
+template <typename S>
+bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
+  return !sys.empty() && cut_batch<S>(b, sys).rows > 0;
+}
+
+template <typename S>
+ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
+  const Cut c = cut_batch<S>(b, sys);
+  if (!c.rows) return fail(OHM_ERR_INVALID, "batch does not fit the resident solve");
+  constexpr int kVecs = 3;
+  // words of every system, then the argument and owner tables
+  std::vector<ResArgs<S, BSys>> args(sys.size());
+  std::vector<int> owner;
+  size_t words = 0;
+  std::vector<size_t> at(sys.size());
+  for (size_t k = 0; k < sys.size(); k++) {
+    const int n = sys[k].geo->n, grid = (n + c.rows - 1) / c.rows;
+    at[k] = words;
+    words += (grid > 1 ? (size_t)kVecs * n * Tagged<S>::kWords : 0) +
+             (size_t)2 * grid * kResSlotWords + 1;
+    for (int g = 0; g < grid; g++) owner.push_back((int)k);
+  }
+  const auto al = [](size_t v) { return (v + 255) & ~size_t(255); };
+  const size_t args_at = al(words * 8), owner_at = args_at + al(sizeof(args[0]) * args.size());
+  void *ws = nullptr;
+  OHM_TRY(resident_ws(b, owner_at + sizeof(int) * owner.size(), &ws));
+  u64 *base = static_cast<u64 *>(ws);
+  int wg = 0;
+  for (size_t k = 0; k < sys.size(); k++) {
+    const BGeo &q = *sys[k].geo;
+    ResArgs<S, BSys> &a = args[k];
+    a = ResArgs<S, BSys>{};
+    a.n = q.n;
+    a.grid = (q.n + c.rows - 1) / c.rows;
+    a.rows = (q.n + a.grid - 1) / a.grid;
+    a.first = wg;
+    wg += a.grid;
+    a.m[0] = ResCsr<S>{q.rowptr, q.col, q.g, q.c, q.sig_re, q.sig_im};
+    a.inv = sys[k].inv;
+    a.x = sys[k].x;
+    a.r = sys[k].r;
+    a.rh = sys[k].rh;
+    a.st = sys[k].st;
+    a.words = base + at[k];
+    a.slots = a.words + (a.grid > 1 ? (size_t)kVecs * q.n * Tagged<S>::kWords : 0);
+    a.outcome = a.slots + (size_t)2 * a.grid * kResSlotWords;
+  }
+  ResArgs<S, BSys> *d_args = reinterpret_cast<ResArgs<S, BSys> *>(static_cast<char *>(ws) + args_at);
+  int *d_owner = reinterpret_cast<int *>(static_cast<char *>(ws) + owner_at);
+  OHM_HIP(hipMemcpyAsync(d_args, args.data(), sizeof(args[0]) * args.size(), hipMemcpyHostToDevice,
+                         b->stream));
+  OHM_HIP(hipMemcpyAsync(d_owner, owner.data(), sizeof(int) * owner.size(), hipMemcpyHostToDevice,
+                         b->stream));
+  hipLaunchKernelGGL(k_clear_words, dim3(grid_for((int64_t)words)), dim3(kBlock), 0, b->stream,
+                     (int64_t)words, base);
+  b->dispatches++;
+  for (size_t q = 0; q + 1 < c.group.size(); q++) {
+    const int k0 = c.group[q], k1 = c.group[q + 1];
+    int rows = 0;
+    for (int k = k0; k < k1; k++) rows = std::max(rows, args[k].rows);
+    const int first = args[k0].first, grid = args[k1 - 1].first + args[k1 - 1].grid - first;
+    const unsigned threads = (unsigned)(rows + 63) / 64 * 64;
+    const unsigned lds = (unsigned)(kVecs * (size_t)rows * sizeof(S));
+    const auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, b->stream, d_args, d_owner, first);
+    };
+    if (c.width == 4)
+      launch(k_batch_resident<S, 4>);
+    else if (c.width == 6)
+      launch(k_batch_resident<S, 6>);
+    else
+      launch(k_batch_resident<S, 8>);
+    OHM_HIP(hipGetLastError());
+    b->dispatches++;
+  }
+  return OHM_OK;
+}
+
+template bool batch_resident_fits<double>(const ohm_backend *,
+                                          const std::vector<BatchSolve<double>> &);
+template bool batch_resident_fits<cx<double>>(const ohm_backend *,
+                                              const std::vector<BatchSolve<cx<double>>> &);
+template ohm_status batch_resident_enqueue<double>(ohm_backend *,
+                                                   const std::vector<BatchSolve<double>> &);
+template ohm_status batch_resident_enqueue<cx<double>>(
+    ohm_backend *, const std::vector<BatchSolve<cx<double>>> &);
+
+}  // namespace ohm

@@ -948,8 +948,7 @@ static ohm_status bicg_drive(ohm_backend *b, const DevCsr &a, const PrecondDev &
   return OHM_OK;
 }
 
-// The backend's workspace for resident solves, at least `bytes` long.
-static ohm_status resident_ws(ohm_backend *b, size_t bytes, void **ws) {
+ohm_status resident_ws(ohm_backend *b, size_t bytes, void **ws) {
   if (b->resident_ws_bytes < bytes) {
     if (b->resident_ws) OHM_HIP(hipFree(b->resident_ws));
     b->resident_ws = nullptr;

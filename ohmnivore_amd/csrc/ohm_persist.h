@@ -29,6 +29,9 @@ struct ResLayout {
 };
 ResLayout resident_layout(const ResGeo &g, const PrecondDev &p, int n, bool f32);
 
+// The backend's workspace for resident solves, at least `bytes` long.
+ohm_status resident_ws(ohm_backend *b, size_t bytes, void **ws);
+
 // Enqueues the solve behind k_init: x, r and r_hat as k_init left them, the
 // workspace `ws` with its first clear_words words zero. On success the state
 // word holds the final status; a solve that could not finish (its workgroups

@@ -1,0 +1,92 @@
+"""Batched solves on resident workgroups (one launch per group of systems)
+against the LU of every system and against the batch engine's own kernels,
+which a check_interval of one's own selects: real and complex, one workgroup
+per system and several, uneven sizes, one and two groups, rows longer than a
+tile, no preconditioner."""
+import numpy as np
+import pytest
+
+import oracle
+from ohmnivore_amd import _native as N
+from ohmnivore_amd import circuit as ir
+from ohmnivore_amd import solver
+from tests.test_gpu_resident import system
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def be():
+    return solver.HipBackend()
+
+
+def lu(a, c, sigma, b):
+    m = ir.CsrMatrix(a.nrows, a.ncols, a.values + sigma * c, a.col_indices, a.row_pointers)
+    if not np.iscomplexobj(m.values):
+        return oracle.sparse_lu_solve(m, b)
+    n = m.nrows  # the complex system as a real one of twice the size
+    rows = np.repeat(np.arange(n), np.diff(m.row_pointers.astype(np.int64)))
+    cols, re, im = m.col_indices.astype(np.int64), m.values.real, m.values.imag
+    big = oracle.from_triplet_arrays(
+        2 * n, 2 * n, np.concatenate([rows, rows, rows + n, rows + n]),
+        np.concatenate([cols, cols + n, cols, cols + n]), np.concatenate([re, -im, im, re]))
+    x = oracle.sparse_lu_solve(big, np.concatenate([b.real, b.imag]))
+    return x[:n] + 1j * x[n:]
+
+
+@pytest.mark.parametrize("complex_", [False, True], ids=["real", "complex"])
+@pytest.mark.parametrize("sizes,per_row,n_dense", [
+    ([65, 300, 512], 3, 0),            # a workgroup each
+    ([513, 40, 1300, 1], 5, 1),        # several, and a system of one row
+    ([640, 641, 1025], 7, 2),
+    ([1600] * 60, 3, 0),               # two groups at 512 rows a workgroup
+    ([33] * 300, 3, 0)],               # more systems than compute units
+    ids=["single", "uneven", "wide", "groups", "many"])
+@pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_NONE], ids=["jacobi", "none"])
+def test_batch_resident_matches_lu(be, complex_, sizes, per_row, n_dense, prec):
+    rng = np.random.default_rng(len(sizes) + per_row)
+    mats = {n: system(n, per_row, n_dense, seed=n) if n > 1 else
+            oracle.from_triplet_arrays(1, 1, np.array([0]), np.array([0]), np.array([2.0]))
+            for n in set(sizes)}
+    caps = {n: np.abs(m.values) * rng.uniform(0.1, 0.2, m.values.shape[0]) *
+            (np.repeat(np.arange(n), np.diff(m.row_pointers.astype(np.int64))) ==
+             m.col_indices) for n, m in mats.items()}
+    systems, rhs = [], []
+    for k, n in enumerate(sizes):
+        m = mats[n]
+        sigma = (1j * (1 + k % 7)) if complex_ else 0.5 * (k % 5)
+        systems.append((m.row_pointers, m.col_indices, m.values, caps[n], sigma))
+        b = rng.standard_normal(n) + (1j * rng.standard_normal(n) if complex_ else 0)
+        rhs.append(b)
+    bt = solver.Batch(be, systems, complex_)
+    prm = dict(tolerance=1e-13, max_iterations=2000)
+    x = bt.solve(np.concatenate(rhs), params=solver.bicgstab_params(**prm), precond=prec)
+    its = [r.iterations for r in bt.last_results]
+    y = bt.solve(np.concatenate(rhs), params=solver.bicgstab_params(check_interval=8, **prm),
+                 precond=prec)
+    assert min(its) >= 1
+    again = bt.solve(np.concatenate(rhs), params=solver.bicgstab_params(**prm), precond=prec)
+    assert again.tobytes() == x.tobytes()
+    for k in list(range(len(sizes)))[:8] + [len(sizes) - 1]:
+        m = mats[sizes[k]]
+        ref = lu(m, caps[sizes[k]], systems[k][4], rhs[k])
+        scale = np.abs(ref).max()
+        # relative residual 1e-13, condition below 10 (row scale up to 7)
+        assert np.abs(bt.split(x)[k] - ref).max() < 1e-11 * scale
+        assert np.abs(bt.split(y)[k] - ref).max() < 1e-11 * scale
+
+
+def test_batch_resident_one_system_fails_alone(be):
+    """A system whose right-hand side is not finite ends by itself; the
+    iteration cap is per system."""
+    m = system(700, 5, 0, seed=3)
+    bt = solver.Batch(be, [(m.row_pointers, m.col_indices, m.values, None, 0.0)] * 3, False)
+    b = np.tile(np.random.default_rng(0).standard_normal(700), 3)
+    b[700] = np.inf
+    x = bt.solve(b, params=solver.bicgstab_params(tolerance=1e-12), raise_on_failure=False)
+    ok = [r.converged for r in bt.last_results]
+    assert ok == [True, False, True]
+    assert bt.split(x)[0].tobytes() == bt.split(x)[2].tobytes()
+    bt.solve(b[:700].repeat(1).tolist() * 3, params=solver.bicgstab_params(
+        tolerance=1e-14, max_iterations=2), raise_on_failure=False)
+    assert [r.iterations for r in bt.last_results] == [2, 2, 2]
