@@ -638,9 +638,14 @@ __global__ __launch_bounds__(64) void k_part_rel(const BandWave *__restrict__ wa
 // p) at index 2p and L_p = x(last row) at 2p+1; their equations
 //   F_p + k_prev L_{p-1} + k_next F_{p+1} = alpha   (bottom-up relation)
 //   L_p + k_prev L_{p-1} + k_next F_{p+1} = alpha   (top-down relation)
-// form a band of half bandwidth 2; solved by LU with partial pivoting (U rows
-// of 5 entries and y to red, x to bnd[(2 pbase + r) * 64 + lane]).
-// blockIdx.x: the partitioned wave.
+// form a band of half bandwidth 2; solved by LU with partial pivoting (per U
+// row the pivot's reciprocal, its 4 other entries and y to red, x to
+// bnd[(2 pbase + r) * 64 + lane]). blockIdx.x: the partitioned wave.
+// One wave walks 2P dependent rows each way, so the time is P times a part's
+// latency. With the rows fetched one step ahead that was the loads' (2.1 us
+// per part); fetched kRedAhead parts ahead, and without a second reciprocal
+// on the way back, it is 1.35 us (78 parts at 61 frequencies 165 -> 105 us).
+constexpr int kRedAhead = 3;
 __global__ __launch_bounds__(64) void k_part_reduce(const BandWave *__restrict__ waves,
                                                     const PartWave *__restrict__ pwaves,
                                                     const cz *__restrict__ rel,
@@ -652,32 +657,36 @@ __global__ __launch_bounds__(64) void k_part_reduce(const BandWave *__restrict__
   if (lane >= q.nf) return;
   const int P = q.nparts, n = 2 * P;
   const size_t rb = (size_t)2 * q.pbase;
-  // band row r of the reduced system: entries for columns r-2 .. r+2
-  auto row = [&](int r, cz (&a)[W], cz &f) {
-#pragma unroll
-    for (int d = 0; d < W; d++) a[d] = cz{0.0, 0.0};
-    f = cz{0.0, 0.0};
+  // row r as stored (alpha, k_prev, k_next); zero past the last row
+  auto fetch = [&](int r, cz (&o)[3]) {
+    o[0] = o[1] = o[2] = cz{0.0, 0.0};
     if (r >= n) return;
     const int p = r >> 1, dir = (r & 1) ? 0 : 1;
-    const cz *o = rel + (size_t)((q.pbase + p) * 2 + dir) * 3 * 64 + lane;
-    f = o[0];
-    const cz kp = p > 0 ? o[64] : cz{0.0, 0.0}, kn = p + 1 < P ? o[128] : cz{0.0, 0.0};
-    if (dir == 1) {  // F_p: L_{p-1} at d 1, F_p at d 2, F_{p+1} at d 4
-      a[1] = kp;
-      a[2] = cz{1.0, 0.0};
-      a[4] = kn;
-    } else {         // L_p: L_{p-1} at d 0, L_p at d 2, F_{p+1} at d 3
-      a[0] = kp;
-      a[2] = cz{1.0, 0.0};
-      a[3] = kn;
+    const cz *s = rel + (size_t)((q.pbase + p) * 2 + dir) * 3 * 64 + lane;
+    o[0] = s[0];
+    if (p > 0) o[1] = s[64];
+    if (p + 1 < P) o[2] = s[128];
+  };
+  // band row r from its stored entries: columns r-2 .. r+2
+  auto band = [&](int r, const cz (&o)[3], cz (&a)[W]) {
+#pragma unroll
+    for (int d = 0; d < W; d++) a[d] = cz{0.0, 0.0};
+    if (r < n) a[2] = cz{1.0, 0.0};
+    if (r & 1) {  // L_p: L_{p-1} at d 0, F_{p+1} at d 3
+      a[0] = o[1];
+      a[3] = o[2];
+    } else {  // F_p: L_{p-1} at d 1, F_{p+1} at d 4
+      a[1] = o[1];
+      a[4] = o[2];
     }
   };
   cz win[KB + 1][W], y[KB + 1];
 #pragma unroll
   for (int r = 0; r <= KB; r++) {
-    cz a[W], f;
-    row(r, a, f);
-    y[r] = f;
+    cz o[3], a[W];
+    fetch(r, o);
+    band(r, o, a);
+    y[r] = o[0];
 #pragma unroll
     for (int c = 0; c < W; c++) win[r][c] = cz{0.0, 0.0};
 #pragma unroll
@@ -687,11 +696,14 @@ __global__ __launch_bounds__(64) void k_part_reduce(const BandWave *__restrict__
     }
   }
   int bad = 0;
-  // the row that enters the window after the next step is loaded one step
-  // ahead, so its loads overlap a step's arithmetic
-  cz na[W], nf;
-  row(KB + 1, na, nf);
-  for (int j = 0; j < n; j++) {
+  // the rows that enter the window after the two steps of part p (2p+3 and
+  // 2p+4) are fetched kRedAhead parts earlier
+  cz in[kRedAhead][2][3];
+#pragma unroll
+  for (int d = 0; d < kRedAhead; d++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) fetch(2 * d + 3 + e, in[d][e]);
+  auto step = [&](int j, const cz (&o)[3]) {
     int pv = 0;
     double best = cabs2(win[0][0]);
 #pragma unroll
@@ -725,8 +737,9 @@ __global__ __launch_bounds__(64) void k_part_reduce(const BandWave *__restrict__
       y[r] = y[r] - l * y[0];
     }
     cz *u = red + ((rb + j) * (W + 1)) * 64 + lane;
+    u[0] = pinv;
 #pragma unroll
-    for (int c = 0; c < W; c++) u[c * 64] = win[0][c];
+    for (int c = 1; c < W; c++) u[c * 64] = win[0][c];
     u[W * 64] = y[0];
 #pragma unroll
     for (int r = 0; r < KB; r++) {
@@ -735,37 +748,53 @@ __global__ __launch_bounds__(64) void k_part_reduce(const BandWave *__restrict__
       win[r][W - 1] = cz{0.0, 0.0};
       y[r] = y[r + 1];
     }
+    band(j + 1 + KB, o, win[KB]);
+    y[KB] = o[0];
+  };
+  for (int p0 = 0; p0 < P; p0 += kRedAhead) {
 #pragma unroll
-    for (int d = 0; d < W; d++) win[KB][d] = na[d];
-    y[KB] = nf;
-    row(j + 2 + KB, na, nf);
+    for (int d = 0; d < kRedAhead; d++) {
+      const int p = p0 + d;
+      if (p < P) {
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          step(2 * p + e, in[d][e]);
+          fetch(2 * (p + kRedAhead) + 3 + e, in[d][e]);
+        }
+      }
+    }
   }
   cz xw[W - 1];
 #pragma unroll
   for (int k = 0; k < W - 1; k++) xw[k] = cz{0.0, 0.0};
-  // the next (lower) row of U and its right-hand side loaded one step ahead
-  cz un[W + 1];
-  auto u_load = [&](int j) {
+  // rows of U, last first, fetched 2 kRedAhead rows ahead
+  constexpr int kAhead = 2 * kRedAhead;
+  cz un[kAhead][W + 1];
+  auto u_load = [&](int j, cz (&v)[W + 1]) {
     if (j < 0) return;
     const cz *u = red + ((rb + j) * (W + 1)) * 64 + lane;
 #pragma unroll
-    for (int c = 0; c <= W; c++) un[c] = u[c * 64];
+    for (int c = 0; c <= W; c++) v[c] = u[c * 64];
   };
-  u_load(n - 1);
-  for (int j = n - 1; j >= 0; j--) {
-    cz u[W + 1];
 #pragma unroll
-    for (int c = 0; c <= W; c++) u[c] = un[c];
-    u_load(j - 1);
-    cz acc = u[W];
+  for (int d = 0; d < kAhead; d++) u_load(n - 1 - d, un[d]);
+  for (int j0 = n - 1; j0 >= 0; j0 -= kAhead) {
 #pragma unroll
-    for (int c = 1; c < W; c++) acc = acc - u[c] * xw[c - 1];
-    const cz d = u[0];
-    const cz xj = cabs2(d) > 0.0 ? acc * cinv(d) : cz{0.0, 0.0};
-    bnd[(rb + j) * 64 + lane] = xj;
+    for (int d = 0; d < kAhead; d++) {
+      const int j = j0 - d;
+      if (j >= 0) {
+        // the newest unknown last: one product on the chain from row to row
+        cz acc = un[d][W];
 #pragma unroll
-    for (int k = W - 2; k > 0; k--) xw[k] = xw[k - 1];
-    xw[0] = xj;
+        for (int c = W - 1; c > 0; c--) acc = acc - un[d][c] * xw[c - 1];
+        const cz xj = acc * un[d][0];
+        u_load(j - kAhead, un[d]);
+        bnd[(rb + j) * 64 + lane] = xj;
+#pragma unroll
+        for (int k = W - 2; k > 0; k--) xw[k] = xw[k - 1];
+        xw[0] = xj;
+      }
+    }
   }
   if (bad) singular[part_sys(waves[q.seg_a], waves[q.seg_b], q, lane)] = 2;
 }
@@ -954,46 +983,54 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
   if (bad) singular[part_sys(qa, qb, q, lane)] = 2;
 }
 
-// One thread per (partitioned wave, lane): the residual terms of every
-// part's first and last row (columns in the neighbouring parts, read from
-// the written x) and the parts' interior sums, in part order, to
-// res[2 sys], beside the circuit's ||b||^2. Identity rows past the lane's
-// own segment have zero residual (x is zero there).
-__global__ void k_part_resid_sum(const BandWave *__restrict__ waves,
-                                 const PartWave *__restrict__ pwaves, int n_waves,
-                                 const PartRef *__restrict__ parts,
-                                 const double *__restrict__ pres, const cz *__restrict__ X,
-                                 double *__restrict__ res) {
+// One workgroup per partitioned wave, a system per lane: wave y takes parts
+// y, y + kResidWaves, ...: the residual terms of a part's first and last row
+// (columns in the neighbouring parts, read from the written x) and its
+// interior sum; the waves' sums are added in order, to res[2 sys], beside the
+// circuit's ||b||^2. Identity rows past the lane's own segment have zero
+// residual (x is zero there). A part is a chain of dependent loads, 1.4 us
+// each when one thread walked all parts of its system; 16 waves share them
+// (78 parts at 61 frequencies 107 -> 20 us).
+constexpr int kResidWaves = 16;
+__global__ __launch_bounds__(64 * kResidWaves) void k_part_resid_sum(
+    const BandWave *__restrict__ waves, const PartWave *__restrict__ pwaves,
+    const PartRef *__restrict__ parts, const double *__restrict__ pres,
+    const cz *__restrict__ X, double *__restrict__ res) {
   constexpr int W = kPartW;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n_waves * 64) return;
-  const PartWave w = pwaves[t / 64];
-  const int lane = t % 64;
-  if (lane >= w.nf) return;
+  __shared__ double sums[kResidWaves][64];
+  const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+  const PartWave w = pwaves[blockIdx.x];
   const bool second = lane >= w.split;
   const BandWave q = waves[second ? w.seg_b : w.seg_a];
   const int l = second ? lane - w.split : lane;
-  const double om = q.omega[l];
-  const cz *Xb = X + w.store_off;
-  const int S = w.nf;
   double rr = 0.0;
-  for (int ip = w.pbase; ip < w.pbase + w.nparts; ip++) {
-    rr += pres[(size_t)ip * 64 + lane];
-    const PartRef pr = parts[ip];
-    for (int e = 0; e < 2; e++) {
-      if (e == 1 && pr.m == 1) break;  // one row: first and last
-      const int64_t i = e == 0 ? pr.s : (int64_t)pr.s + pr.m - 1;
-      if (i >= q.n) continue;
-      cz a[W], bi, xc[W];
-      band_row<W>(q, om, i, a, bi);
+  if (lane < w.nf) {
+    const double om = q.omega[l];
+    const cz *Xb = X + w.store_off;
+    const int S = w.nf;
+    for (int k = wv; k < w.nparts; k += kResidWaves) {
+      const int ip = w.pbase + k;
+      rr += pres[(size_t)ip * 64 + lane];
+      const PartRef pr = parts[ip];
+      for (int e = 0; e < 2; e++) {
+        if (e == 1 && pr.m == 1) break;  // one row: first and last
+        const int64_t i = e == 0 ? pr.s : (int64_t)pr.s + pr.m - 1;
+        if (i >= q.n) continue;
+        cz a[W], bi, xc[W];
+        band_row<W>(q, om, i, a, bi);
 #pragma unroll
-      for (int d = 0; d < W; d++) {
-        const int64_t col = i - 1 + d;
-        xc[d] = col >= 0 && col < q.n ? Xb[col * S + lane] : cz{0.0, 0.0};
+        for (int d = 0; d < W; d++) {
+          const int64_t col = i - 1 + d;
+          xc[d] = col >= 0 && col < q.n ? Xb[col * S + lane] : cz{0.0, 0.0};
+        }
+        rr += resid2<W>(a, bi, xc);
       }
-      rr += resid2<W>(a, bi, xc);
     }
   }
+  sums[wv][lane] = rr;
+  __syncthreads();
+  if (wv > 0 || lane >= w.nf) return;
+  for (int k = 1; k < kResidWaves; k++) rr += sums[k][lane];
   res[2 * (q.sys + l)] = rr;
   res[2 * (q.sys + l) + 1] = q.bnorm2;
 }
@@ -1182,6 +1219,7 @@ struct ohm_ac_plan {
   std::vector<BandWave> waves;  // the resident chunk's wave table
   size_t y_off = 0;             // byte offset of its solutions in the workspace
   int64_t tuned_rows = -1;      // autotuned rows per part (0: one lane per system)
+  bool tune = true;             // the autotuner may time candidates on this plan
   int64_t part_rows = 0;        // rows per part of the last solve
   int chunks = 0;
   int64_t fallback_systems = 0; // systems of the last solve redone in one lane
@@ -1380,8 +1418,29 @@ double direct_budget(ohm_backend *b) {
 // residual ||b - A x|| / ||b|| above which a partitioned system is solved
 // again in one lane
 constexpr double kPartResidMax = 1e-12;
-// rows per part when neither the environment nor the autotuner sets it
-constexpr int64_t kDefaultPartRows = 2048;
+
+// Rows per part when neither the environment nor the autotuner sets it. A
+// sweep that leaves the chip idle takes about 0.6 us per row of a part
+// (relations and part solve, each a dependent chain) and 1.7 us per part of
+// its longest system (the reduced system's chain, the residual's sum), which
+// sqrt(3 rows) balances: one 15,002-row ladder at 61 frequencies 0.25 ms at
+// 192 rows per part (64: 0.46, 512: 0.37, 2,048: 1.23), 192,002 rows 0.96 ms
+// at 768 (256: 1.58, 2,048: 1.43). More waves than the part solve keeps in
+// flight (three on each of 1,024 SIMDs) only add parts, so a larger sweep
+// takes the rows that give this many, up to 2,048 (48 ladders of
+// 1,000-64,000 sections at 101 frequencies: 4.33 ms at 1,536 rows, 4.56 at
+// 768; 25,856 systems: 2,048 rows 21.5 ms, 1,024: 22.3).
+int64_t default_part_rows(const ohm_ac_plan *p, int64_t n_freqs) {
+  constexpr double kWaves = 3 * 1024;
+  double longest = 0.0, lane_rows = 0.0;
+  for (int64_t n : p->n) {
+    longest = std::max(longest, (double)n);
+    lane_rows += (double)n * (double)n_freqs;
+  }
+  const double r = std::max(sqrt(3.0 * longest), std::min(2048.0, lane_rows / (64.0 * kWaves)));
+  const int64_t tile = kPartTile;
+  return std::max<int64_t>(64, ((int64_t)r + tile - 1) / tile * tile);
+}
 
 ohm_status ensure_events(ohm_ac_plan *p) {
   for (auto &e : p->ev)
@@ -1643,8 +1702,8 @@ ohm_status plan_solve_once(ohm_ac_plan *p, int64_t n_freqs, double *const *x, in
                          d_parts, d_bnd, d_ck, dY, p->d_sing, d_pres);
       OHM_HIP(hipGetLastError());
       OHM_HIP(hipEventRecord(ev[3], st));
-      hipLaunchKernelGGL(k_part_resid_sum, dim3((unsigned)((n_pw * 64 + 255) / 256)), dim3(256),
-                         0, st, d_w, d_pw, n_pw, d_parts, d_pres, dY, p->d_res);
+      hipLaunchKernelGGL(k_part_resid_sum, dim3((unsigned)n_pw), dim3(64 * kResidWaves), 0, st,
+                         d_w, d_pw, d_parts, d_pres, dY, p->d_res);
       OHM_HIP(hipGetLastError());
       b->dispatches += 4;
     } else {
@@ -1738,7 +1797,7 @@ ohm_status plan_solve_once(ohm_ac_plan *p, int64_t n_freqs, double *const *x, in
 
 // rows per part: OHM_AC_PART_ROWS, else the autotuned value of this plan
 // (the fastest of the candidates, each timed over two whole sweeps on the
-// plan's first solve), else 2048
+// plan's first solve), else default_part_rows
 ohm_status plan_solve(ohm_ac_plan *p, int64_t n_freqs, const double *freqs, double *const *x,
                       ohm_batch_result *results, double *device_ms) {
   ohm_backend *b = p->b;
@@ -1769,15 +1828,15 @@ ohm_status plan_solve(ohm_ac_plan *p, int64_t n_freqs, const double *freqs, doub
   std::vector<double> omega(n_om, 0.0);
   for (int64_t f = 0; f < n_freqs; f++) omega[f] = 2.0 * M_PI * freqs[f];  // ac.rs:57
   OHM_HIP(hipMemcpyAsync(p->d_omega, omega.data(), sizeof(double) * n_om, hipMemcpyHostToDevice, st));
-  int64_t R = kDefaultPartRows;
+  int64_t R = default_part_rows(p, n_freqs);
   if (const char *env = getenv("OHM_AC_PART_ROWS")) {
     R = atoll(env);
   } else if (p->tuned_rows >= 0) {
     R = p->tuned_rows;
-  } else if (b->autotune && p->B == 1) {
+  } else if (b->autotune && p->tune && p->B == 1) {
     // each candidate timed twice (the faster of the two counts), so that a
     // sweep slowed by its first use of a workspace size does not decide
-    const int64_t cand[] = {0, 1024, 2048, 3072, 4096, 8192};
+    const int64_t cand[] = {0, R / 2, R, R + R / 2, 2 * R, 4 * R};
     double best = 1e300;
     for (int64_t c : cand) {
       double tc = 1e300;
@@ -2007,7 +2066,7 @@ ohm_status ohm_ac_sweep_circuits(ohm_backend *b, int64_t n_circuits, const ohm_a
     }
     ohm_ac_plan *p = nullptr;
     OHM_TRY(plan_build(b, (int64_t)dl.size(), dc.data(), dp, &p));
-    p->tuned_rows = kDefaultPartRows;  // a one-off sweep is not worth tuning
+    p->tune = false;  // a one-off sweep is not worth tuning
     std::vector<ohm_batch_result> dr(dl.size() * std::max<int64_t>(n_freqs, 1));
     double ms = 0.0;
     ohm_status s = plan_solve(p, n_freqs, freqs, dx.data(), dr.data(), &ms);

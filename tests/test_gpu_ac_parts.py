@@ -1,0 +1,54 @@
+"""The partitioned banded AC solve at the edges of its part counts: the
+reduced system fetches a few parts ahead and the residual sum deals the parts
+to 16 waves, so part counts around both (and one part alone) are solved and
+compared with the one-lane LU of whole systems and the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from ohmnivore_amd import circuit as ir
+from ohmnivore_amd import solver
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def be():
+    return solver.HipBackend()
+
+
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 7, 15, 16, 17, 33])
+def test_part_counts(be, parts, monkeypatch):
+    # part boundaries move by at most 16 rows, so 64 k - 31 rows make k parts
+    rows = 64 * parts - 31
+    m = solver.compile(ir.rlc_ladder((rows - 2) // 3, ir.SplitMix64(parts)))
+    assert abs(m.size - rows) <= 3
+    freqs = 10.0 ** np.linspace(0.0, 9.0, 70)     # one full wave and a part of one
+    x = {}
+    for r in ("0", "64"):
+        monkeypatch.setenv("OHM_AC_PART_ROWS", r)
+        res = solver.AcPlan(be, [m]).solve(freqs, keep_x=True)
+        assert float(res.residual_norms.max()) < 1e-12
+        x[r] = res.x[0]
+    scale = np.abs(x["0"]).max(axis=1)
+    assert float((np.abs(x["64"] - x["0"]).max(axis=1) / scale).max()) < 1e-10
+    ref = oracle.ac_sweep(m, freqs)
+    assert np.allclose(x["64"], ref, rtol=1e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize("sections,n_freqs,rows", [
+    (20, 3, 64),          # the smallest part
+    (5000, 61, 224),      # sqrt(3 x 15,002) up to a multiple of 32
+    (5000, 1, 224),
+])
+def test_rows_per_part_rule(be, sections, n_freqs, rows, monkeypatch):
+    monkeypatch.delenv("OHM_AC_PART_ROWS", raising=False)
+    be.set_autotune(False)
+    try:
+        plan = solver.AcPlan(be, [solver.compile(ir.rlc_ladder(sections, ir.SplitMix64(1)))])
+        res = plan.solve(10.0 ** np.linspace(0.0, 9.0, n_freqs))
+    finally:
+        be.set_autotune(True)
+    st = plan.stats()
+    assert st["rows_per_part"] == rows and st["redone_systems"] == 0
+    assert float(res.residual_norms.max()) < 1e-12
