@@ -31,7 +31,7 @@ constexpr int kResBatchGroups = 2;
 template <typename S, int W>
 __global__ __launch_bounds__(kResBatchRows<S>) void k_batch_resident(
     const ResArgs<S, BSys> *__restrict__ args, const int *__restrict__ owner, int first) {
-  using R = Resident<S, BSys, PK_JACOBI, W, false>;
+  using R = Resident<S, BSys, PK_JACOBI, W, 4, false>;
   __shared__ typename R::Shared sh;
   __shared__ ResArgs<S, BSys> a;
   extern __shared__ __align__(16) unsigned char res_lds[];

@@ -1233,6 +1233,7 @@ ohm_status bicg_solve_transpose(ohm_backend *b, DevCsr &a, PrecondDev &p, const 
     DevCsr mlt, mut;
     OHM_TRY(csr_transpose_view(b, p.ml, mlt));
     OHM_TRY(csr_transpose_view(b, p.mu, mut));
+    pt.halo_rows = p.halo_rows;
     pt.ml = mut;  // applied first: M_U^T
     pt.mu = mlt;  // then M_L^T
   }

@@ -127,8 +127,8 @@ __device__ __forceinline__ FusedRow fused_bind(const FusedCsr &m, int r, int n,
 // together, wherever their rows lie, and leave them in LDS at sp; a lane then
 // adds its row's, eight reads at a time. Lanes that walked their own entries
 // one by one waited for two dependent LDS reads per entry, and the whole wave
-// for its longest row (a supply node's): 161 -> 87 us per solve of a 50-stage
-// inverter chain (54 unknowns), 97 -> 65 us at 24 unknowns.
+// for its longest row (a supply node's): 161 -> 84 us per solve of a 50-stage
+// inverter chain (54 unknowns), 97 -> 61 us at 24 unknowns.
 template <bool STAGE>
 __device__ __forceinline__ double fused_spmv(const FusedRow &m, double v, double *sv, double *sp) {
 #pragma clang fp contract(off)

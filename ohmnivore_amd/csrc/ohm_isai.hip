@@ -475,6 +475,7 @@ static ohm_status isai_plan_build(ohm_backend *b, const DevCsr &a, int level, Pr
   // per nonzero, so the two-SpMV form is faster there.
   const char *env = getenv("OHM_ISAI_PRODUCT");
   if (env && atoi(env) != 0) OHM_TRY(build_product(b, p));
+  p.halo_rows = resident_halo_rows(b, a, p.ml, p.mu);
   return OHM_OK;
 }
 

@@ -11,12 +11,16 @@ constexpr int kResThreads = 512;      // most threads of a workgroup (256 regist
 constexpr int kResMaxGrid = 256;      // most workgroups (one per CU)
 constexpr int kResMaxLong = 32;       // rows per matrix beyond the row tile
 constexpr int kResSlotWords = 8;      // 64-bit words of one reduction slot
+constexpr int kResMaxWidth = 8;       // widest row tile
+constexpr int kResHalo = 768;         // most foreign columns a workgroup keeps in LDS
 
 // How a solve is cut: `grid` workgroups of `threads` threads with `rows`
-// consecutive rows each, one per thread, row tiles of `width` entries.
+// consecutive rows each, one per thread, row tiles of `width` entries (the
+// ISAI factors' of `fwidth`).
 // grid == 0: the system does not fit this path.
 struct ResGeo {
-  int grid = 0, threads = 0, rows = 0, width = 0;
+  int grid = 0, threads = 0, rows = 0, width = 0, fwidth = 4;
+  int halo = 1;  // ISAI: 2: the workgroups' spare threads form their halo
 };
 // The geometry of a solve of a x = b with p.
 ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n);

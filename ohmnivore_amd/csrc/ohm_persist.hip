@@ -25,18 +25,27 @@
 //   vector's last read and its next write lies a reduction.
 //
 // Jacobi: 3 reductions per iteration and no other exchange (p_hat and s_hat
-// are formed from r, q and v as they are gathered); ISAI: 3 reductions and 4
-// exchanges. What bounds it is their latency, about 1.7 us a reduction over
-// 20 to 128 workgroups and 1.2 us an exchange, and the 64-bit scalar
-// arithmetic between them. Measured per iteration, pipeline -> here: Jacobi
-// 15.3 -> 3.8 us (102 rows, one workgroup), 21.2 -> 9.7 (10,002), 21.7 -> 12.8
-// (65,540), 24.7 -> 16.6 (129,604); ISAI 29.3 -> 15.1 (2,871), 27.9 -> 15.9
-// (16,388), 35.7 -> 20.7 (65,540), 44.7 -> 25.9 (129,604).
+// are formed from r, q and v as they are gathered). ISAI: the foreign entries
+// of r, q and v are fetched into LDS, once each, by the waves that a reduction
+// leaves idle, so the first product reads LDS alone; the first factor's result
+// and p_hat / s_hat are exchanged, or, where a workgroup's threads past its own
+// rows suffice, their foreign entries are formed a second time by those
+// threads and nothing but the reductions is waited for (2,871 rows: 14.6 us an
+// iteration with four exchanges, 12.1 without). A supply node's row, too long
+// for a thread, has its entries spread over the workgroup's threads: read from
+// memory in every product it cost 1.5 to 3.6 us a product (clock stamps).
+// What bounds an iteration is latency: about 1.7 us a reduction over 20 to 128
+// workgroups, 1.2 us an exchange, 0.4 us a product from LDS and 0.8 us of
+// 64-bit scalar arithmetic. Measured per iteration, pipeline -> here: Jacobi
+// 15.3 -> 3.8 us (102 rows, one workgroup), 21.2 -> 9.7 (10,002), 21.7 -> 12.2
+// (65,540), 25.3 -> 15.8 (129,604); ISAI 29.3 -> 12.5 (2,871), 27.9 -> 15.1
+// (16,388), 29.8 -> 15.9 (32,404), 35.7 -> 19.1 (65,540), 45.4 -> 25.4 (129,604).
 //
 // All workgroups must run at once: the grid has at most one workgroup per
 // compute unit. A wait that lasts longer than kResLimit ends the kernel with
 // nothing written (the outcome word says so to the other workgroups) and the
-// host continues with the pipeline from the state that k_init left.
+// host continues with the pipeline from the state that k_init left; so does a
+// solve that breaks down.
 #include <algorithm>
 #include <mutex>
 
@@ -44,9 +53,10 @@
 
 namespace ohm {
 
-template <typename T, int PK, int W>
+template <typename T, int PK, int W, int WF>
 __global__ __launch_bounds__(kResThreads) void k_bicg_resident(ResArgs<T, SolveState> a) {
-  using R = Resident<T, SolveState, PK, W, PK != PK_ISAI || W <= 6>;
+  constexpr bool kEarly = PK != PK_ISAI && (sizeof(T) == 4 || W <= 6);
+  using R = Resident<T, SolveState, PK, W, WF, kEarly>;
   __shared__ typename R::Shared sh;
   extern __shared__ __align__(16) unsigned char res_lds[];
   R r(a, sh, res_lds);
@@ -71,19 +81,76 @@ ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev
   const DevCsr *ms[3] = {&a, &p.ml, &p.mu};
   const int nm = p.kind == PK_ISAI ? 3 : 1;
   static const int kWidths[3] = {4, 6, 8}, kLong[3] = {2, 2, kResMaxLong};
-  for (int w = 0; w < 3 && !g.width; w++) {
-    bool fits = true;
-    for (int m = 0; m < nm; m++)
-      fits = fits && ms[m]->long_rows[w] >= 0 && ms[m]->long_rows[w] <= kLong[w];
-    if (fits) g.width = kWidths[w];
-  }
-  if (!g.width) return g;
+  const auto width = [&](int m0, int m1) {
+    for (int w = 0; w < 3; w++) {
+      bool fits = true;
+      for (int m = m0; m < m1; m++)
+        fits = fits && ms[m]->long_rows[w] >= 0 && ms[m]->long_rows[w] <= kLong[w];
+      if (fits) return kWidths[w];
+    }
+    return 0;
+  };
+  g.width = width(0, 1);
+  g.fwidth = nm > 1 ? width(1, 3) : 4;
+  if (!g.width || !g.fwidth) return ResGeo();
+  // the factors' rows are about half as long as A's: tiles of 4, or A's width
+  if (g.fwidth > 4) g.width = g.fwidth = std::max(g.width, g.fwidth);
   const int grid = (n + kResThreads - 1) / kResThreads;
   if (grid > std::min(b->num_cu, kResMaxGrid)) return g;
   g.grid = grid;
   g.rows = (n + grid - 1) / grid;
   g.threads = (g.rows + 63) / 64 * 64;
+  // smaller workgroups, whose spare threads form their halo: more of them make
+  // a reduction slower by at most 0.8 us, the four exchanges are worth 2.5
+  if (p.kind == PK_ISAI && grid > 1 && p.halo_rows > 0) {
+    const int hgrid = (n + p.halo_rows - 1) / p.halo_rows;
+    if (hgrid <= std::min(b->num_cu, kResMaxGrid)) {
+      g.grid = hgrid;
+      g.rows = (n + hgrid - 1) / hgrid;
+      g.threads = kResThreads;
+      g.halo = 2;
+    }
+  }
   return g;
+}
+
+// Rows per workgroup, the most whose foreign operands of A's and M_U's rows
+// all find a thread (the kernel's find_halo, over the patterns).
+int resident_halo_rows(const ohm_backend *b, const DevCsr &a, const DevCsr &ml, const DevCsr &mu) {
+  const int n = a.n;
+  if (n <= kResThreads) return 0;
+  const auto tile = [](const DevCsr &m, uint32_t r) {
+    return m.h_rowptr[r + 1] - m.h_rowptr[r] <= (uint32_t)kResMaxWidth;
+  };
+  std::vector<int> seen(n, -1);
+  std::vector<uint32_t> list;
+  for (int rows = kResThreads - 64; rows >= 128; rows -= 64) {
+    const int grid = (n + rows - 1) / rows, even = (n + grid - 1) / grid;
+    if (grid > std::min(b->num_cu, kResMaxGrid)) break;
+    bool fits = true;
+    std::fill(seen.begin(), seen.end(), -1);
+    for (int g = 0; g < grid && fits; g++) {
+      const uint32_t lo = (uint32_t)g * even, hi = (uint32_t)std::min(n, (g + 1) * even);
+      list.clear();
+      const auto join = [&](const DevCsr &m, uint32_t r, bool hat) {
+        if (!tile(m, r)) return;
+        for (uint32_t k = m.h_rowptr[r]; k < m.h_rowptr[r + 1]; k++) {
+          const uint32_t c = m.h_col[k];
+          if ((c >= lo && c < hi) || seen[c] == g || !tile(ml, c) || (hat && !tile(mu, c))) continue;
+          seen[c] = g;
+          list.push_back(c);
+        }
+      };
+      const size_t cap = (size_t)(kResThreads - (int)(hi - lo));
+      for (uint32_t r = lo; r < hi && list.size() <= cap; r++) join(a, r, true);
+      const size_t n_hat = list.size();
+      for (uint32_t r = lo; r < hi && list.size() <= cap; r++) join(mu, r, false);
+      for (size_t i = 0; i < n_hat && list.size() <= cap; i++) join(mu, list[i], false);
+      fits = list.size() <= cap;
+    }
+    if (fits) return rows;
+  }
+  return 0;
 }
 
 ResLayout resident_layout(const ResGeo &g, const PrecondDev &p, int n, bool f32) {
@@ -114,6 +181,7 @@ ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p
   q.n = a.n;
   q.rows = g.rows;
   q.grid = g.grid;
+  q.halo = g.halo;
   q.m[0] = csr(a);
   if (p.kind == PK_ISAI) {
     q.m[1] = csr(p.ml);
@@ -130,23 +198,32 @@ ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p
   q.words = reinterpret_cast<u64 *>(base);
   q.slots = q.words + l.slots;
   q.outcome = q.words + l.outcome;
-  const unsigned lds = (unsigned)((p.kind == PK_ISAI ? 5 : 3) * (size_t)g.rows * sizeof(T));
+  // ISAI: the halo's columns, then the vectors (the hash table before them)
+  const unsigned lds = (unsigned)(p.kind == PK_ISAI
+                                      ? sizeof(uint32_t) * kResHalo +
+                                            std::max(5 * (size_t)(g.rows + kResHalo) * sizeof(T),
+                                                     sizeof(uint32_t) * 8 * kResThreads)
+                                      : 3 * (size_t)g.rows * sizeof(T));
   const auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(g.grid), dim3(g.threads), lds, b->stream, q);
   };
   const auto by_width = [&](auto pk) {
     constexpr int PK = decltype(pk)::value;
     if (g.width == 4)
-      launch(k_bicg_resident<T, PK, 4>);
+      launch(k_bicg_resident<T, PK, 4, 4>);
     else if (g.width == 6)
-      launch(k_bicg_resident<T, PK, 6>);
+      launch(k_bicg_resident<T, PK, 6, 4>);
     else
-      launch(k_bicg_resident<T, PK, 8>);
+      launch(k_bicg_resident<T, PK, 8, 4>);
   };
-  if (p.kind == PK_ISAI)
-    by_width(std::integral_constant<int, PK_ISAI>());
-  else  // without a preconditioner inv is null
+  if (p.kind != PK_ISAI)  // without a preconditioner inv is null
     by_width(std::integral_constant<int, PK_JACOBI>());
+  else if (g.fwidth == 4)
+    by_width(std::integral_constant<int, PK_ISAI>());
+  else if (g.fwidth == 6)
+    launch(k_bicg_resident<T, PK_ISAI, 6, 6>);
+  else
+    launch(k_bicg_resident<T, PK_ISAI, 8, 8>);
   OHM_HIP(hipGetLastError());
   b->dispatches++;
   return OHM_OK;

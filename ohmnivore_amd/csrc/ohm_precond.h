@@ -18,7 +18,12 @@ struct PrecondDev {
   IsaiPlan *plan = nullptr;
   int ilu_sweeps = 5;      // fixed-point ILU(0) sweeps per numeric refresh
   bool has_f32 = false;
+  int halo_rows = 0;       // ISAI: resident_halo_rows of the pattern it was built for
 };
+
+// Rows per workgroup of a resident solve that lets every workgroup form its
+// halo (0: none does). A solve with another pattern is right all the same.
+int resident_halo_rows(const ohm_backend *b, const DevCsr &a, const DevCsr &ml, const DevCsr &mu);
 
 ohm_status precond_build(ohm_backend *b, const DevCsr &a, int kind, int level, PrecondDev &p);
 ohm_status precond_refresh(ohm_backend *b, const DevCsr &a, PrecondDev &p);

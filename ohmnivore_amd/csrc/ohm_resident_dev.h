@@ -33,6 +33,8 @@ template <typename S, typename St>
 struct ResArgs {
   int n, rows;               // unknowns, rows per workgroup
   int first, grid;           // its first workgroup in the launch, and how many
+  int halo;                  // ISAI: 1: foreign operands are fetched into LDS; 2: and the
+                             // foreign results of the factors formed here
   ResCsr<S> m[3];            // A, M_L, M_U
   const S *inv;              // Jacobi inverse diagonal (null: none)
   S *x;
@@ -162,45 +164,52 @@ __device__ __forceinline__ bool res_expired(u64 *outcome, volatile int *dead, u6
   return false;
 }
 
-// A thread's rows of one matrix row each as W entries: `off` is the operand's
-// byte offset, into the workgroup's LDS vector or, where its bit of `far` is
-// set, into the tagged vector.
-template <typename T, int W>
+// A thread's row of one matrix as W entries: `off` is the operand's byte
+// offset, into the workgroup's LDS vector or, where its bit of `far` is set,
+// into the tagged vector. With X set, entry W is the thread's share of a row
+// too long for a tile, summed apart.
+template <typename T, int W, int X>
 struct RowTile {
-  T val[W];
-  uint32_t off[W], far;
+  T val[W + X];
+  uint32_t off[W + X], far;
 };
 
-// kEarly: registers are left to request a product's foreign operands before
-// the reduction that precedes it is complete.
-template <typename T, typename St, int PK, int W, bool kEarly>
+// Row tiles of W entries for A and WF for the factors. kEarly: registers are
+// left to request a product's foreign operands before the reduction that
+// precedes it is complete.
+template <typename T, typename St, int PK, int W, int WF, bool kEarly>
 struct Resident {
   using A = ResAlg<T>;
   static constexpr bool kC = Tr<T>::C;
   static constexpr int kN = kC ? 2 : 1;   // words of a dot product
   static constexpr int kSums = kN + 2;    // sums of one reduction
   static constexpr int kMats = PK == PK_ISAI ? 3 : 1;
+  static constexpr int kX = PK == PK_ISAI ? 1 : 0;  // long rows' shares in the tiles
   static constexpr int kR = 0, kQ = 1, kV = 2, kTmp = 3, kHat = 4;  // vector numbers
   static constexpr int kWaveCap = 16;
   static constexpr uint32_t kWordBytes = 8 * Tagged<T>::kWords;
+  static constexpr int kNoLoads = 0x0f70;  // s_waitcnt: vmcnt 0, the other counters any
 
   struct Shared {
     double sum[2][kSums][kWaveCap];
     double total[2][kSums];
     double part[kResMaxLong][kN][kWaveCap];
     int long_row[kMats][kResMaxLong];
-    int n_long[kMats];
+    int n_long[kMats], kept[kMats];  // kept: the first of them is in the tiles
     int dead, run, given_up[2];
+    int n_slots, n_tmp, n_hat, halo_over;
   };
+  static constexpr uint32_t kEmpty = ~0u;
 
   const ResArgs<T, St> &a;
   Shared &sh;
   char *lv;  // LDS vectors, `rows` entries each
-  int T0, t, lane, wave, waves, g, G, base, cnt;
+  int T0, t, lane, wave, waves, g, G, base, cnt, stride;
   uint32_t round;   // reductions so far
   int8_t long_at[kMats];
-  RowTile<T, W> tiles[kMats];
-  Tagged<T> ahead[2][W];  // words of the foreign operands, requested early
+  RowTile<T, W, kX> tile_a;
+  RowTile<T, WF, kX> tile_f[2];  // M_L, M_U
+  Tagged<T> ahead[2][W];  // Jacobi: words of the foreign operands, requested early
 
   __device__ __forceinline__ Resident(const ResArgs<T, St> &a_, Shared &s_, unsigned char *lv_)
       : a(a_), sh(s_), lv(reinterpret_cast<char *>(lv_)) {
@@ -213,10 +222,12 @@ struct Resident {
     G = a.grid;
     base = g * a.rows;
     cnt = min(a.rows, a.n - base);
+    stride = a.rows + (PK == PK_ISAI ? kResHalo : 0);
+    if (PK == PK_ISAI) lv += sizeof(uint32_t) * kResHalo;
     round = 0;
   }
   __device__ __forceinline__ T near_value(int v, uint32_t off) const {
-    return *reinterpret_cast<const T *>(lv + (uint32_t)(v * a.rows) * (uint32_t)sizeof(T) + off);
+    return *reinterpret_cast<const T *>(lv + (uint32_t)(v * stride) * (uint32_t)sizeof(T) + off);
   }
   // x, its constancy unknown to the compiler: addresses, masks and selected
   // values derived from a row tile are formed at each use (one instruction)
@@ -233,11 +244,12 @@ struct Resident {
   }
   __device__ __forceinline__ bool mine() const { return t < cnt; }
 
-  // publish this thread's entry of vector v
+  // publish this thread's entry of vector v (a halo thread's stays here)
   __device__ __forceinline__ void put(int v, T x, uint32_t tag) {
-    if (!mine()) return;
-    reinterpret_cast<T *>(lv)[v * a.rows + t] = x;
-    if (G > 1) Tagged<T>::put(word(v, (uint32_t)(base + t) * kWordBytes), x, tag);
+    const int halo = v == kTmp ? sh.n_tmp : v == kHat ? sh.n_hat : 0;
+    if (PK == PK_ISAI ? t >= cnt + halo : !mine()) return;
+    reinterpret_cast<T *>(lv)[v * stride + t] = x;
+    if (mine() && G > 1) Tagged<T>::put(word(v, (uint32_t)(base + t) * kWordBytes), x, tag);
   }
 
   __device__ __forceinline__ uint32_t place(uint32_t col, bool &far) const {
@@ -246,150 +258,365 @@ struct Resident {
     return far ? col * kWordBytes : off * (uint32_t)sizeof(T);
   }
 
+  // The halo (ISAI): foreign columns this workgroup reads have a slot in its
+  // LDS vectors, behind its own rows. r, q and v are fetched into every slot
+  // while a reduction is under way, once for all rows that read them. With
+  // a.halo 2 the threads past the own rows also form the foreign entries of
+  // the first factor's result (slots below n_tmp) and of hat (below n_hat),
+  // thread cnt + s slot s, so that neither is waited for.
+  //
+  // While the tiles are built the vectors' place holds a hash table of the
+  // columns: keys, then slots. Their list stays, in front of the vectors.
+  static constexpr int kHash = 2 * kResThreads * 2;
+  __device__ __forceinline__ uint32_t *keys() const { return reinterpret_cast<uint32_t *>(lv); }
+  __device__ __forceinline__ uint32_t *slot_of() const { return keys() + kHash; }
+  __device__ __forceinline__ uint32_t *halo_cols() const { return keys() - kResHalo; }
+  static __device__ __forceinline__ uint32_t bucket(uint32_t col) {
+    return (col * 2654435761u) >> (32 - __builtin_ctz((uint32_t)kHash));
+  }
+  __device__ __forceinline__ bool fits_tile(int m, uint32_t row) const {
+    return a.m[m].rowptr[row + 1] - a.m[m].rowptr[row] <= (uint32_t)(m == 0 ? W : WF);
+  }
+  // The foreign columns of row `row` of matrix m join the halo. A result whose
+  // own row of a factor is not a tile stays an exchange.
+  __device__ __forceinline__ void join(int m, uint32_t row) {
+    if (!fits_tile(m, row)) return;
+    const ResCsr<T> &c = a.m[m];
+    for (uint32_t k = c.rowptr[row]; k < c.rowptr[row + 1]; k++) {
+      const uint32_t col = c.col[k];
+      if (col - (uint32_t)base < (uint32_t)cnt || (m != 1 && !fits_tile(1, col)) ||
+          (m == 0 && !fits_tile(2, col)))
+        continue;
+      uint32_t h = bucket(col);
+      for (int tries = 0;; tries++, h = (h + 1) & (kHash - 1)) {
+        if (tries == kHash) {
+          sh.halo_over = 1;
+          break;
+        }
+        const uint32_t old = atomicCAS(&keys()[h], (unsigned)kEmpty, col);
+        if (old == col) break;
+        if (old != kEmpty) continue;
+        const int s = atomicAdd(&sh.n_slots, 1);
+        if (s < kResHalo) {
+          slot_of()[h] = s;
+          halo_cols()[s] = col;
+        } else {
+          sh.halo_over = 1;
+        }
+        break;
+      }
+    }
+  }
+  __device__ __forceinline__ void clear_halo() {
+    for (int i = t; i < kHash; i += T0) keys()[i] = kEmpty;
+    if (t == 0) sh.n_slots = sh.n_tmp = sh.n_hat = sh.halo_over = 0;
+    __syncthreads();
+  }
+  __device__ __forceinline__ void find_halo() {
+    clear_halo();
+    const int i = t - cnt;
+    if (a.halo > 1) {
+      if (mine()) join(0, base + t);
+      __syncthreads();
+      const int n_hat = sh.n_slots;
+      __syncthreads();
+      if (n_hat <= T0 - cnt) {
+        if (mine())
+          join(2, base + t);
+        else if (i < n_hat)
+          join(2, halo_cols()[i]);
+      }
+      __syncthreads();
+      const int n_tmp = sh.n_slots;
+      __syncthreads();
+      if (n_tmp > T0 - cnt) {
+        clear_halo();  // no thread for each: the results are exchanged
+      } else if (t == 0) {
+        sh.n_hat = n_hat;
+        sh.n_tmp = n_tmp;
+      }
+      __syncthreads();
+    }
+    if (mine())
+      join(1, base + t);
+    else if (i < sh.n_tmp)
+      join(1, halo_cols()[i]);
+    __syncthreads();
+    if (sh.halo_over) clear_halo();  // too many: each row reads its own
+  }
+  // the operand of an entry of matrix m's tile
+  __device__ __forceinline__ uint32_t place_halo(int m, uint32_t col, bool &far) const {
+    const uint32_t off = place(col, far);
+    if (PK != PK_ISAI || !far) return off;
+    uint32_t h = bucket(col);
+    for (int tries = 0; tries < kHash; tries++, h = (h + 1) & (kHash - 1)) {
+      const uint32_t k = keys()[h];
+      if (k == kEmpty) break;
+      if (k != col) continue;
+      const int s = (int)slot_of()[h];
+      if (s >= (m == 0 ? sh.n_hat : m == 2 ? sh.n_tmp : sh.n_slots)) break;
+      far = false;
+      return (uint32_t)(cnt + s) * (uint32_t)sizeof(T);
+    }
+    return off;
+  }
+  // The slots' entries of NV vectors, all with the tag `tag`; by the waves
+  // that have nothing to do in the reduction under way.
+  template <int NV>
+  __device__ __forceinline__ void fetch(const int (&vec)[NV], uint32_t tag) {
+    const int skip = waves > 1 ? 64 : 0, n = sh.n_slots;
+    for (int s = t - skip; s < n; s += T0 - skip) {
+      if (s < 0) break;
+      const uint32_t at = halo_cols()[s] * kWordBytes;
+      Tagged<T> w[NV];
+      int tries = 0;
+      u64 t0 = 0;
+      for (;;) {
+        bool ok = true;
+#pragma unroll
+        for (int v = 0; v < NV; v++) w[v].load(word(vec[v], at));
+#pragma unroll
+        for (int v = 0; v < NV; v++) ok = ok && w[v].is(tag);
+        if (ok || ((++tries & 127) == 0 && res_expired(a.outcome, &sh.dead, t0))) break;
+      }
+#pragma unroll
+      for (int v = 0; v < NV; v++)
+        reinterpret_cast<T *>(lv)[vec[v] * stride + cnt + s] = w[v].get();
+    }
+  }
+
   // This thread's row of matrix m as a tile padded with zeros. A longer row
   // stays in CSR and is summed by the whole workgroup.
-  __device__ __forceinline__ void build(int m) {
+  template <int E>
+  __device__ __forceinline__ void build(int m, RowTile<T, E, kX> &rt) {
     const ResCsr<T> &c = a.m[m];
-    const int row = base + (mine() ? t : 0);
+    int row = base + (mine() ? t : 0);
+    bool has = mine();
+    if (PK == PK_ISAI && !has && m > 0 && t - cnt < (m == 1 ? sh.n_tmp : sh.n_hat)) {
+      row = (int)halo_cols()[t - cnt];
+      has = true;
+    }
     const uint32_t b0 = c.rowptr[row], len = c.rowptr[row + 1] - b0;
-    const bool lg = len > (uint32_t)W;
+    const bool lg = len > (uint32_t)E;
     long_at[m] = -1;
     if (lg && mine()) {
       const int at = atomicAdd(&sh.n_long[m], 1);
       sh.long_row[m][at] = row;
       long_at[m] = (int8_t)at;
     }
-    RowTile<T, W> &rt = tiles[m];
     rt.far = 0;
 #pragma unroll
-    for (int j = 0; j < W; j++) {
-      uint32_t col = (uint32_t)row;
+    for (int j = 0; j < E; j++) {  // padding: zero times an entry of one's own
       T val = zero<T>();
-      if (mine() && !lg && (uint32_t)j < len) {
-        col = c.col[b0 + j];
+      uint32_t off = (uint32_t)(mine() ? t : 0) * (uint32_t)sizeof(T);
+      bool far = false;
+      if (has && !lg && (uint32_t)j < len) {
+        const uint32_t col = c.col[b0 + j];
         val = c.at(b0 + j);
         if (PK == PK_JACOBI && a.inv) val = val * a.inv[col];
+        off = place_halo(m, col, far);
       }
-      bool far;
-      rt.off[j] = place(col, far);
+      rt.off[j] = off;
       rt.val[j] = val;
       if (far) rt.far |= 1u << j;
     }
+    if constexpr (kX) {
+      rt.off[E] = rt.off[0];
+      rt.val[E] = zero<T>();
+    }
+  }
+  // The first row of matrix m too long for a tile, an entry to each thread: a
+  // supply node's, read from memory in every product, was a chain of three
+  // loads and a second exchange that the whole solve waited for.
+  template <int E>
+  __device__ __forceinline__ void keep_long(int m, RowTile<T, E, kX> &rt) {
+    if (!sh.n_long[m]) return;
+    const ResCsr<T> &c = a.m[m];
+    const int row = sh.long_row[m][0];
+    const uint32_t k = c.rowptr[row] + t, e0 = c.rowptr[row + 1];
+    if (e0 - c.rowptr[row] > (uint32_t)T0) return;
+    if (t == 0) sh.kept[m] = 1;
+    if (k >= e0) return;
+    const uint32_t col = c.col[k];
+    bool far;
+    rt.off[E] = place_halo(m, col, far);
+    rt.val[E] = c.at(k);
+    if (PK == PK_JACOBI && a.inv) rt.val[E] = rt.val[E] * a.inv[col];
+    if (far) rt.far |= 1u << E;
   }
 
   // Requests the foreign operands of one row (entries no lane of the wave
   // needs are skipped as one).
   template <int NV, int E>
-  __device__ __forceinline__ void request(const RowTile<T, E> &rt, const int (&vec)[NV],
-                                          Tagged<T> (&w)[NV][E]) const {
+  __device__ __forceinline__ void request(const RowTile<T, E, kX> &rt, const int (&vec)[NV],
+                                          Tagged<T> (&w)[NV][E + kX]) const {
     const uint32_t far = hidden(rt.far);
     if (!__any(far != 0)) return;
 #pragma unroll
-    for (int j = 0; j < E; j++)
+    for (int j = 0; j < E + kX; j++)
       if (far >> j & 1) {
 #pragma unroll
         for (int v = 0; v < NV; v++) w[v][j].load(word(vec[v], rt.off[j]));
       }
   }
 
-  // acc += val . u over E entries whose foreign words `w` were requested
-  // (u = e0, or e0 + coef e1 with two vectors): this workgroup's own entries
-  // from LDS, then the foreign ones in order, spinning until their words
-  // carry the tag. Entries of the other kind take part with a zero, so that
-  // every load is issued before the first is used.
+  // Spins until every foreign word of a row carries its tag. With asked set
+  // the words have been requested once.
   template <int NV, int E>
-  __device__ __forceinline__ T gather(const RowTile<T, E> &rt, const int (&vec)[NV],
-                                      const uint32_t (&tag)[NV], Tagged<T> (&w)[NV][E], T coef,
-                                      T acc) {
+  __device__ __forceinline__ void settle(const RowTile<T, E, kX> &rt, const int (&vec)[NV],
+                                         const uint32_t (&tag)[NV], Tagged<T> (&w)[NV][E + kX],
+                                         bool asked) {
     const uint32_t far = hidden(rt.far);
-    T e[NV][E];
+    const auto missing = [&]() {
+      uint32_t bad = 0;
 #pragma unroll
-    for (int j = 0; j < E; j++) {
+      for (int j = 0; j < E + kX; j++) {
+        bool ok = true;
+#pragma unroll
+        for (int v = 0; v < NV; v++) ok = ok && w[v][j].is(tag[v]);
+        bad |= ok ? 0u : 1u << j;
+      }
+      return bad & far;
+    };
+    int tries = 0;
+    u64 t0 = 0;
+    for (uint32_t bad = asked ? missing() : far; __any(bad != 0); bad = missing()) {
+      if ((++tries & 127) == 0 && res_expired(a.outcome, &sh.dead, t0)) break;
+#pragma unroll
+      for (int j = 0; j < E + kX; j++)
+        if (bad >> j & 1) {
+#pragma unroll
+          for (int v = 0; v < NV; v++) w[v][j].load(word(vec[v], rt.off[j]));
+        }
+    }
+  }
+
+  // The near half of a product: acc += val . u over this workgroup's own
+  // entries (u = e0, or e0 + coef e1 with two vectors), from LDS. Entries of
+  // the other kind take part with a zero, so that every load is issued before
+  // the first is used.
+  template <int NV, int E>
+  __device__ __forceinline__ T near_part(const RowTile<T, E, kX> &rt, const int (&vec)[NV],
+                                         uint32_t far, T coef, T acc, T &share) const {
+    T e[NV][E + kX];
+#pragma unroll
+    for (int j = 0; j < E + kX; j++) {
       const uint32_t off = (far >> j & 1) ? 0u : rt.off[j];
 #pragma unroll
       for (int v = 0; v < NV; v++) e[v][j] = near_value(vec[v], off);
     }
 #pragma unroll
-    for (int j = 0; j < E; j++) {
+    for (int j = 0; j < E + kX; j++) {
       T u = e[0][j];
       if constexpr (NV == 2) u = res_fma<T>(e[1][j], coef, u);
-      acc = res_fma<T>((far >> j & 1) ? zero<T>() : rt.val[j], u, acc);
-    }
-    if (__any(far != 0)) {
-      int tries = 0;
-      u64 t0 = 0;
-      for (;;) {
-        uint32_t bad = 0;
-#pragma unroll
-        for (int j = 0; j < E; j++) {
-          bool ok = true;
-#pragma unroll
-          for (int v = 0; v < NV; v++) ok = ok && w[v][j].is(tag[v]);
-          bad |= ok ? 0u : 1u << j;
-        }
-        bad &= far;
-        if (!__any(bad != 0)) break;
-        if ((++tries & 127) == 0 && res_expired(a.outcome, &sh.dead, t0)) break;
-#pragma unroll
-        for (int j = 0; j < E; j++)
-          if (bad >> j & 1) {
-#pragma unroll
-            for (int v = 0; v < NV; v++) w[v][j].load(word(vec[v], rt.off[j]));
-          }
-      }
-#pragma unroll
-      for (int j = 0; j < E; j++) {
-        T u = w[0][j].get();
-        if constexpr (NV == 2) u = res_fma<T>(w[1][j].get(), coef, u);
-        acc = res_fma<T>((far >> j & 1) ? rt.val[j] : zero<T>(), (far >> j & 1) ? u : zero<T>(), acc);
-      }
+      T &sum = j < E ? acc : share;
+      sum = res_fma<T>((far >> j & 1) ? zero<T>() : rt.val[j], u, sum);
     }
     return acc;
   }
 
+  // acc += val . u over a row's E entries, share += the last one's: this workgroup's own from LDS, then
+  // the foreign ones in order, spinning until their words carry the tag. With
+  // early set their words `w` have been requested.
+  //
+  // No path leaves here with a request open: the compiler would have every
+  // wave wait for it at its next use of the registers, and as the memory
+  // counter is in order, for its own stores of the vector it has just
+  // published, about 1 us a product.
+  template <int NV, int E>
+  __device__ __forceinline__ T gather(const RowTile<T, E, kX> &rt, const int (&vec)[NV],
+                                      const uint32_t (&tag)[NV], Tagged<T> (&w)[NV][E + kX],
+                                      bool early, T coef, T acc, T &share) {
+    const uint32_t far = hidden(rt.far);
+    acc = near_part<NV, E>(rt, vec, far, coef, acc, share);
+    if (!__any(far != 0)) {
+      if (early) __builtin_amdgcn_s_waitcnt(kNoLoads);
+      return acc;
+    }
+    settle<NV, E>(rt, vec, tag, w, early);
+#pragma unroll
+    for (int j = 0; j < E + kX; j++) {
+      T u = w[0][j].get();
+      if constexpr (NV == 2) u = res_fma<T>(w[1][j].get(), coef, u);
+      T &sum = j < E ? acc : share;
+      sum = res_fma<T>((far >> j & 1) ? rt.val[j] : zero<T>(), (far >> j & 1) ? u : zero<T>(), sum);
+    }
+    return acc;
+  }
+
+  template <int M>
+  __device__ __forceinline__ auto &tile() {
+    if constexpr (M == 0)
+      return tile_a;
+    else
+      return tile_f[M - 1];
+  }
+
   // Requests the foreign operands of the product that follows a reduction.
-  __device__ __forceinline__ void look_ahead(int m, const int (&vec)[2]) {
-    if constexpr (kEarly) request<2, W>(tiles[m], vec, ahead);
+  // They have been sent before the sums of the reduction, so the waves that
+  // have nothing to do in it wait for them here.
+  __device__ __forceinline__ void look_ahead(const int (&vec)[2], uint32_t t0, uint32_t t1) {
+    if constexpr (PK == PK_ISAI) {
+      const int v1[1] = {kV};
+      if (G == 1) return;
+      if (t0 == t1)
+        fetch<2>(vec, t0);
+      else  // r is there
+        fetch<1>(v1, t1);
+    } else if constexpr (kEarly) {
+      request<2, W>(tile_a, vec, ahead);
+      const uint32_t tag[2] = {t0, t1};
+      if (wave != 0) settle<2, W>(tile_a, vec, tag, ahead, true);
+    }
+  }
+
+  // This thread's share of a long row that is not in the tiles.
+  template <int NV>
+  __device__ __forceinline__ T long_share(const ResCsr<T> &c, int row, const int (&vec)[NV],
+                                          const uint32_t (&tag)[NV], T coef) {
+    const uint32_t b0 = c.rowptr[row], e0 = c.rowptr[row + 1];
+    T acc = zero<T>(), none = acc;
+    for (uint32_t k = b0 + t; k < e0; k += 4 * T0) {
+      RowTile<T, 4, kX> rt;
+      rt.far = 0;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const uint32_t kk = k + u * T0;
+        const bool in = kk < e0;
+        const uint32_t cc = in ? c.col[kk] : (uint32_t)base;
+        rt.val[u] = in ? c.at(kk) : zero<T>();
+        if (PK == PK_JACOBI && a.inv) rt.val[u] = rt.val[u] * a.inv[cc];
+        bool far;
+        rt.off[u] = place(cc, far);
+        if (far) rt.far |= 1u << u;
+      }
+      if constexpr (kX) {
+        rt.val[4] = zero<T>();
+        rt.off[4] = 0;
+      }
+      Tagged<T> w[NV][4 + kX];
+      acc = gather<NV, 4>(rt, vec, tag, w, false, coef, acc, none);
+    }
+    return acc;
   }
 
   // This thread's entry of M u, u of one or two vectors; a product of two
   // vectors follows look_ahead.
-  template <int NV>
-  __device__ __forceinline__ T product(int m, const int (&vec)[NV], const uint32_t (&tag)[NV],
-                                       T coef) {
-    T y;
-    if constexpr (NV == 2 && kEarly) {
-      y = gather<NV, W>(tiles[m], vec, tag, ahead, coef, zero<T>());
+  template <int m, int NV>
+  __device__ __forceinline__ T product(const int (&vec)[NV], const uint32_t (&tag)[NV], T coef) {
+    constexpr int E = m == 0 ? W : WF;
+    T y, share = zero<T>();
+    if constexpr (NV == 2 && kEarly && PK != PK_ISAI) {
+      y = gather<NV, E>(tile<m>(), vec, tag, ahead, true, coef, zero<T>(), share);
     } else {
-      Tagged<T> w[NV][W];
-      request<NV, W>(tiles[m], vec, w);
-      y = gather<NV, W>(tiles[m], vec, tag, w, coef, zero<T>());
+      Tagged<T> w[NV][E + kX];
+      y = gather<NV, E>(tile<m>(), vec, tag, w, false, coef, zero<T>(), share);
     }
     const int nl = sh.n_long[m];
     if (!nl) return y;
-    const ResCsr<T> &c = a.m[m];
     for (int i = 0; i < nl; i++) {
-      const int row = sh.long_row[m][i];
-      const uint32_t b0 = c.rowptr[row], e0 = c.rowptr[row + 1];
-      T acc = zero<T>();
-      for (uint32_t k = b0 + t; k < e0; k += 4 * T0) {
-        RowTile<T, 4> rt;
-        rt.far = 0;
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const uint32_t kk = k + u * T0;
-          const bool in = kk < e0;
-          const uint32_t cc = in ? c.col[kk] : (uint32_t)base;
-          rt.val[u] = in ? c.at(kk) : zero<T>();
-          if (PK == PK_JACOBI && a.inv) rt.val[u] = rt.val[u] * a.inv[cc];
-          bool far;
-          rt.off[u] = place(cc, far);
-          if (far) rt.far |= 1u << u;
-        }
-        Tagged<T> w[NV][4];
-        request<NV, 4>(rt, vec, w);
-        acc = gather<NV, 4>(rt, vec, tag, w, coef, acc);
-      }
+      T acc = share;
+      if (i > 0 || !sh.kept[m]) acc = long_share<NV>(a.m[m], sh.long_row[m][i], vec, tag, coef);
       const double re = wave_sum(re_of(acc)), im = kC ? wave_sum(im_of(acc)) : 0.0;
       if (lane == 0) {
         sh.part[i][0][wave] = re;
@@ -404,6 +631,7 @@ struct Resident {
       y = mk<T>(s[0], s[1]);
     }
     __syncthreads();
+    __builtin_amdgcn_s_waitcnt(kNoLoads);
     return y;
   }
 
@@ -522,7 +750,7 @@ struct Resident {
       sh.dead = 0;
       sh.run = a.st->status == ST_RUNNING && res_load(a.outcome) == RES_OPEN;
 #pragma unroll
-      for (int m = 0; m < kMats; m++) sh.n_long[m] = 0;
+      for (int m = 0; m < kMats; m++) sh.n_long[m] = sh.kept[m] = 0;
     }
     for (int i = t; i < 2 * kSums * kWaveCap; i += T0) (&sh.sum[0][0][0])[i] = 0.0;
     __syncthreads();
@@ -534,8 +762,19 @@ struct Resident {
     // product (v, t); zero in threads without one
     T x = zero<T>(), r = x, rh = x, q = x, p = x, ph = x, v = x, u = x, hat = x, out = x,
       inv = mk<T>(1.0, 0.0);
-#pragma unroll
-    for (int m = 0; m < kMats; m++) build(m);
+    if constexpr (PK == PK_ISAI) find_halo();
+    build<W>(0, tile_a);
+    if constexpr (PK == PK_ISAI) {
+      build<WF>(1, tile_f[0]);
+      build<WF>(2, tile_f[1]);
+    }
+    if constexpr (kX) {
+      __syncthreads();
+      keep_long<W>(0, tile_a);
+      keep_long<WF>(1, tile_f[0]);
+      keep_long<WF>(2, tile_f[1]);
+      __syncthreads();  // the table's place is the vectors' now
+    }
     if (mine()) {
       const int row = base + t;
       x = a.x[row];
@@ -549,11 +788,10 @@ struct Resident {
     dot(rh, r, d);
     d[kN] = norm2(r);
     d[kN + 1] = 0.0;
-    constexpr int kFirst = PK == PK_ISAI ? 1 : 0;  // the matrix that meets r, q and v
     const int tmpv[1] = {kTmp}, hatv[1] = {kHat};
     int two[2] = {kR, kQ};
     double part = deposit(d);
-    look_ahead(kFirst, two);
+    look_ahead(two, 1, 1);
     if (!collect(part, d)) return;
     A rhr = value(d), rho = alg_make<A>(1.0, 0.0), alpha = rho, omega = rho;
     double rr = d[kN], res2 = rr;
@@ -582,17 +820,20 @@ struct Resident {
 #pragma unroll 1
       for (int half = 0; half < 2; half++) {
         const uint32_t tag2[2] = {rt, half ? rt + 1 : rt}, tag1[1] = {rt + 1 + half};
+        // everything older than the reduction is done: said here, where it costs
+        // nothing, so that no later use of a register waits for it
+        __builtin_amdgcn_s_waitcnt(kNoLoads);
         u = res_fma<T>(half ? v : q, coef, r);
         if constexpr (PK == PK_ISAI) {
-          put(kTmp, product<2>(1, two, tag2, coef), tag1[0]);
+          put(kTmp, product<1, 2>(two, tag2, coef), tag1[0]);
           __syncthreads();
-          hat = product<1>(2, tmpv, tag1, coef);
+          hat = product<2, 1>(tmpv, tag1, coef);
           put(kHat, hat, tag1[0]);
           __syncthreads();
-          out = product<1>(0, hatv, tag1, coef);
+          out = product<0, 1>(hatv, tag1, coef);
         } else {
           hat = inv * u;
-          out = product<2>(0, two, tag2, coef);
+          out = product<0, 2>(two, tag2, coef);
         }
         if (half == 0) put(kV, out, tag1[0]);
         dot(half ? out : rh, half ? u : out, d);
@@ -600,7 +841,7 @@ struct Resident {
         d[kN + 1] = norm2(u);
         part = deposit(d);
         two[1] = kV;
-        if (half == 0) look_ahead(kFirst, two);
+        if (half == 0) look_ahead(two, rt, rt + 1);
         if (!collect(part, d)) return;
         if (half == 0) {
           p = u;
@@ -644,20 +885,25 @@ struct Resident {
       d[kN + 1] = 0.0;
       part = deposit(d);
       two[1] = kQ;
-      look_ahead(kFirst, two);
+      look_ahead(two, rt, rt);
       if (!collect(part, d)) return;
       rhr = value(d);
       rr = d[kN];
       res2 = rr;
     }
     // Workgroup 0 decides that the solve stands; nobody writes x before that.
+    // A breakdown does not stand: it hangs on rounding, so the pipeline, which
+    // sums in another order, has the last word on it.
+    const bool broke = status == ST_BRK_RHO || status == ST_BRK_RV || status == ST_BRK_TT ||
+                       status == ST_BRK_OMEGA;
     if (t == 0) {
       u64 o = RES_OPEN;
       if (g == 0) {
         u64 want = RES_OPEN;
-        __hip_atomic_compare_exchange_strong(a.outcome, &want, (u64)RES_COMMIT, __ATOMIC_RELAXED,
+        const u64 end = broke ? RES_ABORT : RES_COMMIT;
+        __hip_atomic_compare_exchange_strong(a.outcome, &want, end, __ATOMIC_RELAXED,
                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        o = want == RES_OPEN ? (u64)RES_COMMIT : want;
+        o = want == RES_OPEN ? end : want;
       } else {
         u64 t0 = 0;
         int tries = 0;

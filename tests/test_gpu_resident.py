@@ -113,3 +113,61 @@ def test_resident_stops(be):
             solve(be, a, np.where(np.arange(700) == 690, np.inf, b), N.PREC_JACOBI, **kw)
     x, st = solve(be, a, np.zeros(700), N.PREC_JACOBI)
     assert not x.any() and st.iterations == 0
+
+
+def mesh(rows, cols, seed, supply=0):
+    """A rows x cols five-point mesh of random conductances to neighbours and
+    ground; with supply set the last unknown joins that many of the nodes."""
+    rng = np.random.default_rng(seed)
+    n = rows * cols
+    idx = np.arange(n).reshape(rows, cols)
+    pairs = [(idx[:, :-1].ravel(), idx[:, 1:].ravel()), (idx[:-1].ravel(), idx[1:].ravel())]
+    if supply:
+        at = rng.choice(n, supply, replace=False)
+        pairs.append((np.full(supply, n), at))
+        n += 1
+    r, c, v = [], [], []
+    for p, q in pairs:
+        g = rng.uniform(0.5, 1.5, p.shape[0])
+        r += [p, q]
+        c += [q, p]
+        v += [-g, -g]
+    r, c, v = (np.concatenate(k) for k in (r, c, v))
+    diag = rng.uniform(0.5, 1.5, n)
+    np.add.at(diag, r, -v)
+    return oracle.from_triplet_arrays(n, n, np.concatenate([r, np.arange(n)]),
+                                      np.concatenate([c, np.arange(n)]),
+                                      np.concatenate([v, diag]))
+
+
+# The workgroups' halo under ISAI: formed by their spare threads (narrow
+# meshes), fetched only (wide ones), with a row too long for a thread, and with
+# a preconditioner of another pattern, whose halo finds no threads. The
+# condition number is below 20 and the residual below 1e-12: errors below 1e-10.
+@pytest.mark.parametrize("rows,cols,supply", [(33, 16, 0), (61, 47, 0), (61, 47, 20),
+                                              (90, 70, 600), (70, 130, 5), (12, 700, 0)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32_ir"])
+def test_resident_halo(be, rows, cols, supply, precision):
+    a = mesh(rows, cols, seed=rows, supply=supply)
+    b = np.random.default_rng(cols).standard_normal(a.nrows)
+    ref = oracle.sparse_lu_solve(a, b)
+    x, st = solve(be, a, b, N.PREC_ISAI, precision=precision, **TOL)
+    assert st.residual_norm < 1e-12
+    assert np.abs(x - ref).max() < 1e-10 * np.abs(ref).max()
+    y, _ = solve(be, a, b, N.PREC_ISAI, precision=precision, **TOL)
+    assert y.tobytes() == x.tobytes()
+
+
+def test_resident_halo_of_another_pattern(be):
+    a, other = mesh(61, 47, seed=1), system(61 * 47, 7, 0, seed=2)
+    b = np.random.default_rng(3).standard_normal(a.nrows)
+    for m, q in ((a, other), (other, a)):
+        dm = be.upload_matrix(m.values, m.col_indices, m.row_pointers, m.nrows)
+        dq = be.upload_matrix(q.values, q.col_indices, q.row_pointers, q.nrows)
+        p = be.preconditioner(dq, N.PREC_ISAI)
+        bb, xx = be.new_buffer(m.nrows), be.new_buffer(m.nrows)
+        be.upload_vec(b, bb)
+        st = be.bicgstab(dm, bb, xx, p, solver.bicgstab_params(**TOL))
+        ref = oracle.sparse_lu_solve(m, b)
+        assert st.residual_norm < 1e-12
+        assert np.abs(be.download_vec(xx) - ref).max() < 1e-10 * np.abs(ref).max()
