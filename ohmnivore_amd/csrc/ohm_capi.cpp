@@ -133,8 +133,8 @@ ohm_status ohm_backend_counters(const ohm_backend *b, int64_t *dispatches, int64
 }
 
 // ------------------------------------------------------------ buffers ----
-ohm_status ohm_buffer_new(ohm_backend *b, size_t n, ohm_buffer **out) {
-  if (!b || !out) return fail(OHM_ERR_INVALID, "null handle");
+// A buffer whose clearing the stream may still have before it.
+static ohm_status buffer_new(ohm_backend *b, size_t n, ohm_buffer **out) {
   ohm_buffer *buf = new ohm_buffer();
   buf->owner = b;
   buf->n = n;
@@ -143,9 +143,15 @@ ohm_status ohm_buffer_new(ohm_backend *b, size_t n, ohm_buffer **out) {
     delete buf;
     return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
   }
-  OHM_HIP(hipMemsetAsync(buf->d, 0, sizeof(double) * (n ? n : 1), b->stream));
-  OHM_HIP(hipStreamSynchronize(b->stream));
   *out = buf;
+  OHM_HIP(hipMemsetAsync(buf->d, 0, sizeof(double) * (n ? n : 1), b->stream));
+  return OHM_OK;
+}
+
+ohm_status ohm_buffer_new(ohm_backend *b, size_t n, ohm_buffer **out) {
+  if (!b || !out) return fail(OHM_ERR_INVALID, "null handle");
+  OHM_TRY(buffer_new(b, n, out));
+  OHM_HIP(hipStreamSynchronize(b->stream));
   return OHM_OK;
 }
 
@@ -197,22 +203,30 @@ static ohm_status validate_csr(const uint32_t *col, const uint32_t *rowptr, size
   return OHM_OK;
 }
 
-ohm_status ohm_upload_matrix(ohm_backend *b, const double *values, const uint32_t *col_indices,
-                             const uint32_t *row_pointers, size_t n, size_t nnz,
-                             ohm_matrix **out) {
+static ohm_status upload_matrix(ohm_backend *b, const double *values, const uint32_t *col_indices,
+                                const uint32_t *row_pointers, size_t n, size_t nnz,
+                                ohm_matrix **out, std::vector<char> *stage) {
   if (!b || !out || !row_pointers || (nnz && (!col_indices || !values)))
     return fail(OHM_ERR_INVALID, "null handle");
   OHM_TRY(validate_csr(col_indices, row_pointers, n, nnz));
   ohm_matrix *m = new ohm_matrix();
   m->owner = b;
-  ohm_status s = csr_upload(b, m->csr, values, col_indices, row_pointers, (int)n, (int64_t)nnz);
+  ohm_status s = csr_upload(b, m->csr, values, col_indices, row_pointers, (int)n, (int64_t)nnz,
+                            stage);
   if (s != OHM_OK) {
+    (void)hipStreamSynchronize(b->stream);
     csr_free(m->csr);
     delete m;
     return s;
   }
   *out = m;
   return OHM_OK;
+}
+
+ohm_status ohm_upload_matrix(ohm_backend *b, const double *values, const uint32_t *col_indices,
+                             const uint32_t *row_pointers, size_t n, size_t nnz,
+                             ohm_matrix **out) {
+  return upload_matrix(b, values, col_indices, row_pointers, n, nnz, out, nullptr);
 }
 
 void ohm_matrix_free(ohm_matrix *m) {
@@ -371,13 +385,12 @@ ohm_status ohm_scale(ohm_backend *b, double alpha, ohm_buffer *x) {
 }
 
 // ------------------------------------------------------ preconditioners --
-ohm_status ohm_precond_create(ohm_backend *b, const ohm_matrix *a, int kind, int level,
+static ohm_status precond_new(ohm_backend *b, const ohm_matrix *a, int kind, int level, bool wait,
                               ohm_precond **out) {
-  if (!b || !a || !out) return fail(OHM_ERR_INVALID, "null handle");
   ohm_precond *p = new ohm_precond();
   p->owner = b;
   ohm_status s = precond_build(b, a->csr, kind, level, p->dev);
-  if (s == OHM_OK) {
+  if (s == OHM_OK && wait) {
     hipError_t e = hipStreamSynchronize(b->stream);
     if (e != hipSuccess) s = hip_fail(e, "hipStreamSynchronize", __FILE__, __LINE__);
   }
@@ -388,6 +401,12 @@ ohm_status ohm_precond_create(ohm_backend *b, const ohm_matrix *a, int kind, int
   }
   *out = p;
   return OHM_OK;
+}
+
+ohm_status ohm_precond_create(ohm_backend *b, const ohm_matrix *a, int kind, int level,
+                              ohm_precond **out) {
+  if (!b || !a || !out) return fail(OHM_ERR_INVALID, "null handle");
+  return precond_new(b, a, kind, level, true, out);
 }
 
 ohm_status ohm_precond_update(ohm_backend *b, ohm_precond *p, const ohm_matrix *a) {
@@ -478,14 +497,10 @@ static ohm_status run_bicgstab(ohm_backend *b, DevCsr &a, PrecondDev &pd, const 
   else
     s = bicg_solve_f64(b, a, pd, rhs, x, o, out);
   OHM_HIP(hipEventRecord(b->ev1, b->stream));
-  OHM_HIP(hipEventSynchronize(b->ev1));
   if (result) {
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, b->ev0, b->ev1);
     result->iterations = out.iters;
     result->refinements = refinements;
     result->fp64_fallback = out.fp64_fallback ? 1 : 0;
-    result->device_ms = ms;
     result->dispatches = b->dispatches - d0;
     result->readbacks = out.polls;
     double rel = NAN;
@@ -498,6 +513,13 @@ static ohm_status run_bicgstab(ohm_backend *b, DevCsr &a, PrecondDev &pd, const 
       g_last_error = keep;
     }
     result->residual_norm = rel;
+    // read behind the residual's own wait for the stream
+    float ms = 0.f;
+    OHM_HIP(hipEventSynchronize(b->ev1));
+    (void)hipEventElapsedTime(&ms, b->ev0, b->ev1);
+    result->device_ms = ms;
+  } else {
+    OHM_HIP(hipEventSynchronize(b->ev1));
   }
   return s;
 }
@@ -579,17 +601,26 @@ ohm_status ohm_solve_real(ohm_backend *b, size_t n, size_t nnz, const double *va
                           const ohm_bicgstab_params *params, ohm_bicgstab_result *result) {
   if (!b) return fail(OHM_ERR_INVALID, "null backend");
   if (n == 0) return OHM_OK;  // src/solver/gpu.rs:117-119
+  // Uploads are enqueued and not waited for: their sources (the caller's
+  // arrays and `stage`) last until the stream has been waited for below, and
+  // everything that reads them is on the same stream. 41 unknowns: 213 -> 153 us.
+  std::vector<char> stage;
   ohm_matrix *a = nullptr;
-  OHM_TRY(ohm_upload_matrix(b, values, col_indices, row_pointers, n, nnz, &a));
+  OHM_TRY(upload_matrix(b, values, col_indices, row_pointers, n, nnz, &a, &stage));
   ohm_buffer *bb = nullptr, *xx = nullptr;
   ohm_precond *p = nullptr;
-  ohm_status s = ohm_buffer_new(b, n, &bb);
-  if (s == OHM_OK) s = ohm_buffer_new(b, n, &xx);
-  if (s == OHM_OK) s = ohm_upload_vec(b, rhs, n, bb);
-  if (s == OHM_OK && params && params->warm_start) s = ohm_upload_vec(b, x, n, xx);
-  if (s == OHM_OK) s = ohm_precond_create(b, a, precond, 1, &p);
+  const auto enqueue_vec = [&](const double *v, ohm_buffer *to) -> ohm_status {
+    OHM_HIP(hipMemcpyAsync(to->d, v, sizeof(double) * n, hipMemcpyHostToDevice, b->stream));
+    return OHM_OK;
+  };
+  ohm_status s = buffer_new(b, n, &bb);
+  if (s == OHM_OK) s = buffer_new(b, n, &xx);
+  if (s == OHM_OK) s = enqueue_vec(rhs, bb);
+  if (s == OHM_OK && params && params->warm_start) s = enqueue_vec(x, xx);
+  if (s == OHM_OK) s = precond_new(b, a, precond, 1, false, &p);
   if (s == OHM_OK) s = ohm_bicgstab(b, a, bb, xx, p, params, result);
   if (s == OHM_OK) s = ohm_download_vec(b, xx, x, n);
+  if (s != OHM_OK) (void)hipStreamSynchronize(b->stream);
   std::string keep = g_last_error;
   ohm_precond_free(p);
   ohm_buffer_free(bb);

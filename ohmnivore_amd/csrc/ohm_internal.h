@@ -118,6 +118,13 @@ struct DevCsr {
   // rows with more than 4, 6 and 8 entries, of A and of A^T (-1: not counted)
   int long_rows[3] = {-1, -1, -1}, t_long_rows[3] = {-1, -1, -1};
   std::vector<uint32_t> h_rowptr, h_col; // host copy of the pattern
+  // small matrices: the one allocation that holds rowptr, col, val, diag_pos
+  // and the first block table
+  char *pack = nullptr;
+  size_t pack_bytes = 0;
+  bool packed(const void *p) const {
+    return pack && (const char *)p >= pack && (const char *)p < pack + pack_bytes;
+  }
 };
 
 }  // namespace ohm
@@ -188,8 +195,10 @@ void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]);
 ohm_status csr_autotune(ohm_backend *b, DevCsr &m, int *rows_out, int *nnz_out,
                         bool fused = false);
 ohm_status stream_timed(ohm_backend *b, int64_t bytes, int mode, int reps, double &avg_ms);
+// With stage set the copies may still be reading val, col, rowptr and *stage
+// when it returns; the caller keeps them until the stream is synchronised.
 ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32_t *col,
-                      const uint32_t *rowptr, int n, int64_t nnz);
+                      const uint32_t *rowptr, int n, int64_t nnz, std::vector<char> *stage = nullptr);
 void csr_free(DevCsr &m);
 ohm_status csr_ensure_f32(ohm_backend *b, DevCsr &m);
 ohm_status csr_ensure_transpose(ohm_backend *b, DevCsr &m);

@@ -11,6 +11,7 @@
 // Every launch is a bandwidth-bound pass: bytes = nnz*(V+4) + 4(n+1) + 2nV.
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 #include "ohm_spmv.h"
 
@@ -246,8 +247,13 @@ ohm_status csr_ensure_f32(ohm_backend *b, DevCsr &m) {
   return OHM_OK;
 }
 
+// Up to this size a matrix is one allocation and one copy: a 41-unknown one
+// costs 2 calls instead of 10, and the device one small copy instead of five;
+// beyond it the extra pass over the host arrays is no longer small beside them.
+constexpr size_t kPackBytes = 64 * 1024;
+
 ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32_t *col,
-                      const uint32_t *rowptr, int n, int64_t nnz) {
+                      const uint32_t *rowptr, int n, int64_t nnz, std::vector<char> *stage) {
   m.n = n;
   m.nnz = nnz;
   m.h_rowptr.assign(rowptr, rowptr + n + 1);
@@ -266,24 +272,50 @@ ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32
         diag[r] = (int32_t)k;
         break;
       }
-  size_t nz = (size_t)std::max<int64_t>(nnz, 1);
-  OHM_HIP(hipMalloc(&m.rowptr, sizeof(uint32_t) * (n + 1)));
-  OHM_HIP(hipMalloc(&m.col, sizeof(uint32_t) * nz));
-  OHM_HIP(hipMalloc(&m.val, sizeof(double) * nz));
-  OHM_HIP(hipMalloc(&m.blocks, sizeof(uint32_t) * blocks.size()));
-  OHM_HIP(hipMalloc(&m.diag_pos, sizeof(int32_t) * diag.size()));
-  OHM_HIP(hipMemcpyAsync(m.rowptr, rowptr, sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice,
-                         b->stream));
-  if (nnz > 0) {
-    OHM_HIP(hipMemcpyAsync(m.col, col, sizeof(uint32_t) * nnz, hipMemcpyHostToDevice, b->stream));
-    if (val)
-      OHM_HIP(hipMemcpyAsync(m.val, val, sizeof(double) * nnz, hipMemcpyHostToDevice, b->stream));
+  const size_t nz = (size_t)std::max<int64_t>(nnz, 1);
+  struct Part {
+    void **dev;
+    const void *src;
+    size_t bytes, copy;
+  };
+  const Part parts[5] = {
+      {(void **)&m.val, val, sizeof(double) * nz, val ? sizeof(double) * nnz : 0},
+      {(void **)&m.rowptr, rowptr, sizeof(uint32_t) * (n + 1), sizeof(uint32_t) * (n + 1)},
+      {(void **)&m.col, col, sizeof(uint32_t) * nz, sizeof(uint32_t) * nnz},
+      {(void **)&m.blocks, blocks.data(), sizeof(uint32_t) * blocks.size(),
+       sizeof(uint32_t) * blocks.size()},
+      {(void **)&m.diag_pos, diag.data(), sizeof(int32_t) * diag.size(),
+       sizeof(int32_t) * diag.size()}};
+  const auto al = [](size_t v) { return (v + 15) & ~size_t(15); };
+  size_t total = 0;
+  for (const Part &p : parts) total += al(p.bytes);
+  std::vector<char> local;
+  std::vector<char> &hold = stage ? *stage : local;
+  if (total <= kPackBytes) {
+    hold.assign(total, 0);
+    OHM_HIP(hipMalloc(&m.pack, total));
+    m.pack_bytes = total;
+    size_t off = 0;
+    for (const Part &p : parts) {
+      *p.dev = m.pack + off;
+      if (p.copy) std::memcpy(hold.data() + off, p.src, p.copy);
+      off += al(p.bytes);
+    }
+    OHM_HIP(hipMemcpyAsync(m.pack, hold.data(), total, hipMemcpyHostToDevice, b->stream));
+  } else {
+    // the tables made here are copied from `hold`, which outlives them
+    hold.resize(al(parts[3].bytes) + parts[4].bytes);
+    std::memcpy(hold.data(), parts[3].src, parts[3].bytes);
+    std::memcpy(hold.data() + al(parts[3].bytes), parts[4].src, parts[4].bytes);
+    for (const Part &p : parts) {
+      OHM_HIP(hipMalloc(p.dev, p.bytes));
+      const void *src = &p == &parts[3]   ? hold.data()
+                        : &p == &parts[4] ? hold.data() + al(parts[3].bytes)
+                                          : p.src;
+      if (p.copy) OHM_HIP(hipMemcpyAsync(*p.dev, src, p.copy, hipMemcpyHostToDevice, b->stream));
+    }
   }
-  OHM_HIP(hipMemcpyAsync(m.blocks, blocks.data(), sizeof(uint32_t) * blocks.size(),
-                         hipMemcpyHostToDevice, b->stream));
-  OHM_HIP(hipMemcpyAsync(m.diag_pos, diag.data(), sizeof(int32_t) * diag.size(),
-                         hipMemcpyHostToDevice, b->stream));
-  OHM_HIP(hipStreamSynchronize(b->stream));
+  if (!stage) OHM_HIP(hipStreamSynchronize(b->stream));
   return OHM_OK;
 }
 
@@ -366,7 +398,7 @@ ohm_status csr_autotune(ohm_backend *b, DevCsr &m, int *rows_out, int *nnz_out, 
       uint32_t *nb = nullptr;
       OHM_HIP(hipMalloc(&nb, sizeof(uint32_t) * blocks.size()));
       OHM_HIP(hipMemcpy(nb, blocks.data(), sizeof(uint32_t) * blocks.size(), hipMemcpyHostToDevice));
-      if (m.blocks) OHM_HIP(hipFree(m.blocks));
+      if (m.blocks && !m.packed(m.blocks)) OHM_HIP(hipFree(m.blocks));
       m.blocks = nb;
       m.n_blocks = (int)bounds.size() - 1;
       m.tuned_rows = e.second.first;
@@ -445,7 +477,7 @@ ohm_status csr_autotune(ohm_backend *b, DevCsr &m, int *rows_out, int *nnz_out, 
     (void)hipMemcpyAsync(nb, best_blocks.data(), sizeof(uint32_t) * best_blocks.size(),
                          hipMemcpyHostToDevice, b->stream);
     (void)hipStreamSynchronize(b->stream);
-    if (m.blocks) (void)hipFree(m.blocks);
+    if (m.blocks && !m.packed(m.blocks)) (void)hipFree(m.blocks);
     m.blocks = nb;
     m.n_blocks = (int)best_blocks.size() / 2 - 1;
     m.tuned_rows = best_r;
@@ -470,7 +502,8 @@ void csr_free(DevCsr &m) {
   void *ptrs[] = {m.rowptr, m.col,    m.val,   m.val32, m.blocks,  m.diag_pos,
                   m.t_rowptr, m.t_col, m.t_src, m.t_blocks, m.t_val};
   for (void *p : ptrs)
-    if (p) (void)hipFree(p);
+    if (p && !m.packed(p)) (void)hipFree(p);
+  if (m.pack) (void)hipFree(m.pack);
   m = DevCsr();
 }
 

@@ -171,3 +171,22 @@ def test_resident_halo_of_another_pattern(be):
         ref = oracle.sparse_lu_solve(m, b)
         assert st.residual_norm < 1e-12
         assert np.abs(be.download_vec(xx) - ref).max() < 1e-10 * np.abs(ref).max()
+
+
+# A matrix of at most 64 KiB is one allocation and one copy (here up to about
+# 1,480 rows), a larger one an allocation an array; either is tuned and solved.
+@pytest.mark.parametrize("n", [1, 2, 41, 1400, 1600])
+@pytest.mark.parametrize("prec", [N.PREC_NONE, N.PREC_JACOBI, N.PREC_ISAI],
+                         ids=["none", "jacobi", "isai"])
+def test_one_shot_solve(be, n, prec):
+    a = system(n, 3, 0, seed=n)
+    b = np.random.default_rng(n).standard_normal(n)
+    ref = oracle.sparse_lu_solve(a, b)
+    s = solver.GpuSolver(be, precond=prec, params=solver.bicgstab_params(**TOL))
+    assert np.abs(s.solve_real(a, b) - ref).max() < 1e-11 * np.abs(ref).max()
+    m = be.upload_matrix(a.values, a.col_indices, a.row_pointers, n)
+    m.autotune()
+    x, y = be.new_buffer(n), be.new_buffer(n)
+    be.upload_vec(b, x)
+    be.spmv(m, x, y)
+    assert np.allclose(be.download_vec(y), oracle.spmv(a, b), rtol=1e-13, atol=1e-13)
