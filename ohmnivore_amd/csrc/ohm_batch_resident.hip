@@ -13,7 +13,7 @@
 // tiles of six entries spill). Systems that do not fit the chip together go in
 // groups, one launch after another; with more than kResBatchGroups of them the
 // nine launches, or a workgroup per system, do as well. Measured, ten
-// backward-Euler steps of 8 x 16,388 real rows 41.8 -> 17.8 ms (1,150
+// backward-Euler steps of 8 x 16,388 real rows 39.7 -> 15.0 ms (1,150
 // iterations); 21 x 1,847 complex rows 16.6 -> 7.3 ms (375 to 481 iterations).
 #include <algorithm>
 
