@@ -342,7 +342,10 @@ struct Resident {
     else if (i < sh.n_tmp)
       join(1, halo_cols()[i]);
     __syncthreads();
-    if (sh.halo_over) clear_halo();  // too many: each row reads its own
+    // clear_halo resets the flag: every thread reads it before any goes on
+    const int over = sh.halo_over;
+    __syncthreads();
+    if (over) clear_halo();  // too many: each row reads its own
   }
   // the operand of an entry of matrix m's tile
   __device__ __forceinline__ uint32_t place_halo(int m, uint32_t col, bool &far) const {

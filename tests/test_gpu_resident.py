@@ -190,3 +190,21 @@ def test_one_shot_solve(be, n, prec):
     be.upload_vec(b, x)
     be.spmv(m, x, y)
     assert np.allclose(be.download_vec(y), oracle.spmv(a, b), rtol=1e-13, atol=1e-13)
+
+
+@pytest.mark.parametrize("rows,cols", [(60, 50), (120, 120)])
+def test_resident_isai_of_unordered_numbering(be, rows, cols):
+    """Node numbers in random order: a workgroup's rows of M_L have more
+    foreign columns (1,700 at 120 x 120) than its halo holds (768), so every
+    row reads its own. Condition and residual as in test_resident_halo."""
+    m = mesh(rows, cols, seed=rows)
+    perm = np.random.default_rng(cols).permutation(m.nrows)
+    r = np.repeat(np.arange(m.nrows), np.diff(m.row_pointers.astype(np.int64)))
+    a = oracle.from_triplet_arrays(m.nrows, m.nrows, perm[r], perm[m.col_indices], m.values)
+    b = np.random.default_rng(rows).standard_normal(a.nrows)
+    ref = oracle.sparse_lu_solve(a, b)
+    x, st = solve(be, a, b, N.PREC_ISAI, **TOL)
+    assert st.residual_norm < 1e-12
+    assert np.abs(x - ref).max() < 1e-10 * np.abs(ref).max()
+    y, _ = solve(be, a, b, N.PREC_ISAI, **TOL)
+    assert y.tobytes() == x.tobytes()
