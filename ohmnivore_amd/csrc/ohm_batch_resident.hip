@@ -62,10 +62,10 @@ struct Cut {
 template <typename S>
 Cut cut_batch(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
   Cut c;
-  static const int kWidths[3] = {4, 6, 8}, kLong[3] = {2, 2, kResMaxLong};
+  static const int kWidths[3] = {4, 6, 8};
   for (int w = 0; w < 3 && !c.width; w++) {
     bool fits = true;
-    for (const auto &s : sys) fits = fits && s.long_rows[w] <= kLong[w];
+    for (const auto &s : sys) fits = fits && s.long_rows[w] <= kResMaxLong;
     if (fits) c.width = kWidths[w];
   }
   if (!c.width) return c;

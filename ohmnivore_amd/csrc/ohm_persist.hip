@@ -72,20 +72,20 @@ void resident_unlock() { g_resident_mu.unlock(); }
 // registers, and the pipeline, whose launches then carry enough work, is
 // faster (ISAI at 160,004 rows: 59 us per iteration against 49, at 262,148 97
 // against 62), so the path ends at 512 rows for each compute unit. Tiles of
-// 4, 6 or 8 entries; a few longer rows (a supply node's) are summed by their
-// whole workgroup, more of them belong to the pipeline's row blocks. Up to 64
+// 4, 6 or 8 entries; kResMaxLong longer rows (a supply node's) are summed by
+// their whole workgroup, more of them belong to the pipeline's row blocks. Up to 64
 // unknowns the one-wave solve needs no workgroup barriers at all.
 ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n) {
   ResGeo g;
   if (n <= 64 || (p.kind == PK_ISAI && p.mm.rowptr)) return g;
   const DevCsr *ms[3] = {&a, &p.ml, &p.mu};
   const int nm = p.kind == PK_ISAI ? 3 : 1;
-  static const int kWidths[3] = {4, 6, 8}, kLong[3] = {2, 2, kResMaxLong};
+  static const int kWidths[3] = {4, 6, 8};
   const auto width = [&](int m0, int m1) {
     for (int w = 0; w < 3; w++) {
       bool fits = true;
       for (int m = m0; m < m1; m++)
-        fits = fits && ms[m]->long_rows[w] >= 0 && ms[m]->long_rows[w] <= kLong[w];
+        fits = fits && ms[m]->long_rows[w] >= 0 && ms[m]->long_rows[w] <= kResMaxLong;
       if (fits) return kWidths[w];
     }
     return 0;

@@ -208,3 +208,16 @@ def test_resident_isai_of_unordered_numbering(be, rows, cols):
     assert np.abs(x - ref).max() < 1e-10 * np.abs(ref).max()
     y, _ = solve(be, a, b, N.PREC_ISAI, **TOL)
     assert y.tobytes() == x.tobytes()
+
+
+@pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_ISAI], ids=["jacobi", "isai"])
+def test_more_than_two_long_rows_take_the_pipeline(be, prec):
+    """Rows longer than a tile are summed one after the other by their whole
+    workgroup: two of them stay in the resident solve, three do not."""
+    b = np.random.default_rng(8).standard_normal(2000)
+    for n_long, resident in ((2, True), (3, False)):
+        a = system(2000, 3, n_long, seed=n_long)
+        ref = oracle.sparse_lu_solve(a, b)
+        x, st = solve(be, a, b, prec, **TOL)
+        assert np.abs(x - ref).max() < 1e-11 * np.abs(ref).max()
+        assert (st.dispatches < 8) == resident
