@@ -966,9 +966,10 @@ template <typename T>
 static ohm_status bicg_core(ohm_backend *b, const DevCsr &a, const PrecondDev &p, const T *rhs,
                             Workspace<T> &w, const BicgOpts &o, BicgOut &out) {
   Parts pp;
-  const ResGeo geo = resident_geometry(b, a, p, a.n);
+  constexpr bool f32 = std::is_same<T, float>::value;
+  const ResGeo geo = resident_geometry(b, a, p, a.n, f32);
   if (geo.grid && o.check_interval <= 0) {
-    const ResLayout lay = resident_layout(geo, p, a.n, std::is_same<T, float>::value);
+    const ResLayout lay = resident_layout(geo, p, a.n, f32);
     void *ws = w.resident;
     if (!ws) OHM_TRY(resident_ws(b, lay.bytes, &ws));
     if (!w.resident || lay.bytes <= w.resident_bytes) {
@@ -1022,7 +1023,7 @@ ohm_status captured_create(ohm_backend *b, const DevCsr &a, const PrecondDev &p,
   hipError_t e = hipMalloc(&c->vecs, sizeof(double) * stride * kWsVectors);
   if (e == hipSuccess) e = hipMalloc(&c->st, sizeof(SolveState));
   if (e == hipSuccess) e = hipMalloc(&c->partials, sizeof(double) * parts_doubles(a, p, n));
-  c->geo = resident_geometry(b, a, p, n);
+  c->geo = resident_geometry(b, a, p, n, false);
   if (e == hipSuccess && c->geo.grid)
     e = hipMalloc(&c->resident, resident_layout(c->geo, p, n, false).bytes);
   if (e != hipSuccess) {

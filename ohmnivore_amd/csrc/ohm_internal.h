@@ -117,6 +117,7 @@ struct DevCsr {
   int per = kSpmvNnzPerBlock / kBlock;  // entries per thread: tuned_nnz / kBlock
   // rows with more than 4, 6 and 8 entries, of A and of A^T (-1: not counted)
   int long_rows[3] = {-1, -1, -1}, t_long_rows[3] = {-1, -1, -1};
+  int scatter = 0, t_scatter = 0;  // scattered_lines of A and of A^T
   std::vector<uint32_t> h_rowptr, h_col; // host copy of the pattern
   // small matrices: the one allocation that holds rowptr, col, val, diag_pos
   // and the first block table
@@ -190,6 +191,13 @@ void build_spmv_blocks(const uint32_t *rowptr, int n, std::vector<uint32_t> &blo
 int spmv_default_per(const uint32_t *rowptr, int n);
 // Rows with more than 4, 6 and 8 entries.
 void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]);
+// How many separate places 64 neighbouring rows read far from themselves:
+// groups of 8 columns outside the rows' own block of (nearly) 512, averaged over
+// eight samples; 0 up to kScatterRows rows, which no rule tells apart. Up to 20
+// for a mesh numbered row by row, 125 for a ladder and 250 for a mesh with
+// node numbers in random order.
+constexpr int kScatterRows = 3500;
+int scattered_lines(const uint32_t *rowptr, const uint32_t *col, int n);
 // Pick the fastest (rows_cap, nnz_cap) for m by timing each candidate.
 // fused: m is applied by the fused BiCGSTAB kernels (keep 256-row blocks)
 ohm_status csr_autotune(ohm_backend *b, DevCsr &m, int *rows_out, int *nnz_out,

@@ -74,6 +74,28 @@ void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]) {
   }
 }
 
+int scattered_lines(const uint32_t *rowptr, const uint32_t *col, int n) {
+  if (n <= kScatterRows) return 0;
+  constexpr int kSamples = 8, kRows = 64, kBlockRows = 512;
+  const int blocks = (n + kBlockRows - 1) / kBlockRows, rows = (n + blocks - 1) / blocks;
+  std::vector<uint32_t> lines;
+  size_t total = 0;
+  for (int s = 0; s < kSamples; s++) {
+    const int r0 = (int)((int64_t)(n - kRows) * s / (kSamples - 1));
+    lines.clear();
+    for (int r = r0; r < r0 + kRows; r++) {
+      const uint32_t lo = (uint32_t)(r / rows * rows);
+      // a longer row's entries are read together
+      const uint32_t end = std::min(rowptr[r + 1], rowptr[r] + 8);
+      for (uint32_t k = rowptr[r]; k < end; k++)
+        if (col[k] - lo >= (uint32_t)rows) lines.push_back(col[k] / 8);
+    }
+    std::sort(lines.begin(), lines.end());
+    total += std::unique(lines.begin(), lines.end()) - lines.begin();
+  }
+  return (int)(total / kSamples);
+}
+
 // Device block table: (first row, first nonzero) of every block boundary, so
 // a workgroup reads its row and nonzero ranges with one 16-byte scalar load.
 std::vector<uint32_t> spmv_block_pairs(const uint32_t *rowptr, const std::vector<uint32_t> &bounds) {
@@ -259,6 +281,7 @@ ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32
   m.h_rowptr.assign(rowptr, rowptr + n + 1);
   m.h_col.assign(col, col + nnz);
   count_long_rows(rowptr, n, m.long_rows);
+  m.scatter = scattered_lines(rowptr, col, n);
   std::vector<uint32_t> bounds;
   m.per = spmv_default_per(rowptr, n);
   m.tuned_nnz = m.per * kBlock;
@@ -334,6 +357,7 @@ ohm_status csr_ensure_transpose(ohm_backend *b, DevCsr &m) {
     }
   std::vector<uint32_t> bounds;
   count_long_rows(trp.data(), n, m.t_long_rows);
+  m.t_scatter = scattered_lines(trp.data(), tcol.data(), n);
   build_spmv_blocks(trp.data(), n, bounds);
   m.t_n_blocks = (int)bounds.size() - 1;
   const std::vector<uint32_t> blocks = spmv_block_pairs(trp.data(), bounds);
@@ -373,6 +397,7 @@ ohm_status csr_transpose_view(ohm_backend *b, DevCsr &m, DevCsr &view) {
   view.blocks = m.t_blocks;
   view.n_blocks = m.t_n_blocks;
   std::copy(m.t_long_rows, m.t_long_rows + 3, view.long_rows);
+  view.scatter = m.t_scatter;
   return OHM_OK;
 }
 

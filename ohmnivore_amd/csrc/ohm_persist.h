@@ -26,8 +26,9 @@ struct ResGeo {
   int grid = 0, threads = 0, rows = 0, width = 0, fwidth = 4;
   int halo = 1;  // ISAI: 2: the workgroups' spare threads form their halo
 };
-// The geometry of a solve of a x = b with p.
-ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n);
+// The geometry of a solve of a x = b with p, in 32 bits with f32 set.
+ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n,
+                         bool f32);
 
 // Workspace of one solve, cleared before it: tagged vectors, reduction slots
 // and the outcome word.

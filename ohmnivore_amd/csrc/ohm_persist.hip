@@ -75,11 +75,27 @@ void resident_unlock() { g_resident_mu.unlock(); }
 // 4, 6 or 8 entries; kResMaxLong longer rows (a supply node's) are summed by
 // their whole workgroup, more of them belong to the pipeline's row blocks. Up to 64
 // unknowns the one-wave solve needs no workgroup barriers at all.
-ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n) {
+//
+// A matrix whose rows read far and apart costs a word's round trip for each
+// entry, and more workgroups more of them. Per iteration in 64 bits, pipeline
+// -> here: Jacobi, a mesh in random order 21.9 -> 21.2 us at 3,969 rows (170
+// places), 21.0 -> 22.0 at 5,929 (198), 24.7 -> 27.4 at 60,025 (249); three random
+// neighbours a row 26.6 -> 26.2 at 60,000 (186). ISAI, over the three matrices: a
+// ladder in random order 28.7 -> 27.4 us at 3,200 rows, 29.2 -> 30.2 at 4,000
+// (230), 35.6 -> 45.3 at 60,000 (295); with its own pattern for the factors 28.6 ->
+// 13.6 at 6,000 (218; the halo holds), 28.0 -> 29.4 at 9,000 (223). In 32 bits a
+// value is one word and the resident solve stays the faster one (1.05 to 2 times).
+ResGeo resident_geometry(const ohm_backend *b, const DevCsr &a, const PrecondDev &p, int n,
+                         bool f32) {
   ResGeo g;
   if (n <= 64 || (p.kind == PK_ISAI && p.mm.rowptr)) return g;
   const DevCsr *ms[3] = {&a, &p.ml, &p.mu};
   const int nm = p.kind == PK_ISAI ? 3 : 1;
+  if (!f32) {
+    int places = 0;
+    for (int m = 0; m < nm; m++) places += ms[m]->scatter;
+    if (places > (nm == 1 ? 185 : 220)) return g;
+  }
   static const int kWidths[3] = {4, 6, 8};
   const auto width = [&](int m0, int m1) {
     for (int w = 0; w < 3; w++) {

@@ -278,11 +278,14 @@ struct Resident {
     return a.m[m].rowptr[row + 1] - a.m[m].rowptr[row] <= (uint32_t)(m == 0 ? W : WF);
   }
   // The foreign columns of row `row` of matrix m join the halo. A result whose
-  // own row of a factor is not a tile stays an exchange.
+  // own row of a factor is not a tile stays an exchange. Once the halo is too
+  // large nothing more joins: it will be dropped, and a full table takes a
+  // probe of every bucket per column.
   __device__ __forceinline__ void join(int m, uint32_t row) {
     if (!fits_tile(m, row)) return;
     const ResCsr<T> &c = a.m[m];
-    for (uint32_t k = c.rowptr[row]; k < c.rowptr[row + 1]; k++) {
+    const volatile int *over = &sh.halo_over;
+    for (uint32_t k = c.rowptr[row]; k < c.rowptr[row + 1] && !*over; k++) {
       const uint32_t col = c.col[k];
       if (col - (uint32_t)base < (uint32_t)cnt || (m != 1 && !fits_tile(1, col)) ||
           (m == 0 && !fits_tile(2, col)))

@@ -192,22 +192,49 @@ def test_one_shot_solve(be, n, prec):
     assert np.allclose(be.download_vec(y), oracle.spmv(a, b), rtol=1e-13, atol=1e-13)
 
 
-@pytest.mark.parametrize("rows,cols", [(60, 50), (120, 120)])
-def test_resident_isai_of_unordered_numbering(be, rows, cols):
+def shuffled(a, seed):
+    """a with its unknowns numbered in random order."""
+    perm = np.random.default_rng(seed).permutation(a.nrows)
+    r = np.repeat(np.arange(a.nrows), np.diff(a.row_pointers.astype(np.int64)))
+    return oracle.from_triplet_arrays(a.nrows, a.nrows, perm[r], perm[a.col_indices], a.values)
+
+
+@pytest.mark.parametrize("make,level", [(lambda: system(3000, 3, 0, seed=1), 1),
+                                        (lambda: mesh(60, 50, seed=2), 0)], ids=["ladder", "mesh"])
+def test_resident_isai_of_unordered_numbering(be, make, level):
     """Node numbers in random order: a workgroup's rows of M_L have more
-    foreign columns (1,700 at 120 x 120) than its halo holds (768), so every
-    row reads its own. Condition and residual as in test_resident_halo."""
-    m = mesh(rows, cols, seed=rows)
-    perm = np.random.default_rng(cols).permutation(m.nrows)
-    r = np.repeat(np.arange(m.nrows), np.diff(m.row_pointers.astype(np.int64)))
-    a = oracle.from_triplet_arrays(m.nrows, m.nrows, perm[r], perm[m.col_indices], m.values)
-    b = np.random.default_rng(rows).standard_normal(a.nrows)
+    foreign columns (1,035 and 1,268) than its halo holds (768), so every row
+    reads its own. Condition and residual as in test_resident_halo."""
+    a = shuffled(make(), seed=1)
+    b = np.random.default_rng(a.nrows).standard_normal(a.nrows)
     ref = oracle.sparse_lu_solve(a, b)
-    x, st = solve(be, a, b, N.PREC_ISAI, **TOL)
-    assert st.residual_norm < 1e-12
-    assert np.abs(x - ref).max() < 1e-10 * np.abs(ref).max()
-    y, _ = solve(be, a, b, N.PREC_ISAI, **TOL)
-    assert y.tobytes() == x.tobytes()
+    m = be.upload_matrix(a.values, a.col_indices, a.row_pointers, a.nrows)
+    p = be.preconditioner(m, N.PREC_ISAI, level)
+    bb, out = be.new_buffer(a.nrows), []
+    be.upload_vec(b, bb)
+    for _ in range(2):
+        xx = be.new_buffer(a.nrows)
+        st = be.bicgstab(m, bb, xx, p, solver.bicgstab_params(**TOL))
+        assert st.dispatches < 8 and st.residual_norm < 1e-12
+        out.append(be.download_vec(xx))
+    assert np.abs(out[0] - ref).max() < 1e-10 * np.abs(ref).max()
+    assert out[0].tobytes() == out[1].tobytes()
+
+
+@pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_ISAI], ids=["jacobi", "isai"])
+def test_large_unordered_systems_take_the_pipeline(be, prec):
+    """Beyond a few thousand rows a matrix in random order is the pipeline's in
+    64 bits; in row order, or in 32 bits, the resident solve's."""
+    a = mesh(100, 90, seed=4) if prec == N.PREC_JACOBI else system(9000, 3, 0, seed=4)
+    b = np.random.default_rng(5).standard_normal(a.nrows)
+    for q, resident in ((a, True), (shuffled(a, 6), False)):
+        ref = oracle.sparse_lu_solve(q, b)
+        x, st = solve(be, q, b, prec, **TOL)
+        assert np.abs(x - ref).max() < 1e-10 * np.abs(ref).max()
+        assert (st.dispatches < 8) == resident
+        y, st = solve(be, q, b, prec, precision="fp32_ir", **TOL)
+        assert np.abs(y - ref).max() < 1e-10 * np.abs(ref).max()
+        assert st.dispatches < 40
 
 
 @pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_ISAI], ids=["jacobi", "isai"])
