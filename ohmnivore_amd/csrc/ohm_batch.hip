@@ -860,6 +860,7 @@ struct ohm_batch {
   std::vector<void *> allocs;    // patterns and values
   std::vector<int64_t> h_nnz;    // per system
   std::vector<int> h_long;       // per system: rows with more than 4, 6 and 8 entries
+  std::vector<char> res_tables;  // of the resident solve under way, while they upload
   bool has_f32 = false;
   bool jac64_valid = false, jac32_valid = false;  // Jacobi inverses match the current sigmas
   // workspaces: 10 vectors each (x r rh p v s t ph sh inv) + rhs/ax scratch
@@ -1038,7 +1039,7 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
     if (o.check_interval <= 0 && batch_resident_fits<S>(b, list)) {
       ResidentGuard guard(true);
       enqueue_start<S>(bt, w, (int)tab.size(), ia);
-      OHM_TRY(batch_resident_enqueue<S>(b, list));
+      OHM_TRY(batch_resident_enqueue<S>(b, list, bt->res_tables));
       OHM_HIP(hipMemcpyAsync(bt->h_sys, bt->d_sys, sizeof(BSys) * K, hipMemcpyDeviceToHost,
                              stream));
       OHM_HIP(hipStreamSynchronize(stream));

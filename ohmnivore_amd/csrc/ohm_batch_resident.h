@@ -25,8 +25,10 @@ bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> 
 
 // Enqueues the solves. A system that could not finish stays RUNNING with its
 // vectors untouched. The caller holds the resident lock until the launches
-// are done.
+// are done, and keeps `tables`, which the upload may still be reading, until
+// it has waited for the stream.
 template <typename S>
-ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys);
+ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys,
+                                  std::vector<char> &tables);
 
 }  // namespace ohm

@@ -16,6 +16,7 @@
 // backward-Euler steps of 8 x 16,388 real rows 39.7 -> 15.0 ms (1,150
 // iterations); 21 x 1,847 complex rows 16.6 -> 7.3 ms (375 to 481 iterations).
 #include <algorithm>
+#include <new>
 
 #include "ohm_batch_resident.h"
 #include "ohm_resident_dev.h"
@@ -105,36 +106,39 @@ bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> 
 }
 
 template <typename S>
-ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
+ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys,
+                                  std::vector<char> &tables) {
   const Cut c = cut_batch<S>(b, sys);
   if (!c.rows) return fail(OHM_ERR_INVALID, "batch does not fit the resident solve");
   constexpr int kVecs = 3;
-  // words of every system, then the argument and owner tables
-  std::vector<ResArgs<S, BSys>> args(sys.size());
-  std::vector<int> owner;
-  size_t words = 0;
+  // words of every system, then the argument and owner tables (one upload)
+  size_t words = 0, wgs = 0;
   std::vector<size_t> at(sys.size());
   for (size_t k = 0; k < sys.size(); k++) {
     const int n = sys[k].geo->n, grid = (n + c.rows - 1) / c.rows;
     at[k] = words;
     words += (grid > 1 ? (size_t)kVecs * n * Tagged<S>::kWords : 0) +
              (size_t)2 * grid * kResSlotWords + 1;
-    for (int g = 0; g < grid; g++) owner.push_back((int)k);
+    wgs += grid;
   }
+  using Args = ResArgs<S, BSys>;
   const auto al = [](size_t v) { return (v + 255) & ~size_t(255); };
-  const size_t args_at = al(words * 8), owner_at = args_at + al(sizeof(args[0]) * args.size());
+  const size_t args_at = al(words * 8), owner_off = al(sizeof(Args) * sys.size());
+  tables.resize(owner_off + sizeof(int) * wgs);
   void *ws = nullptr;
-  OHM_TRY(resident_ws(b, owner_at + sizeof(int) * owner.size(), &ws));
+  OHM_TRY(resident_ws(b, args_at + tables.size(), &ws));
   u64 *base = static_cast<u64 *>(ws);
+  Args *args = reinterpret_cast<Args *>(tables.data());
+  int *owner = reinterpret_cast<int *>(tables.data() + owner_off);
   int wg = 0;
   for (size_t k = 0; k < sys.size(); k++) {
     const BGeo &q = *sys[k].geo;
-    ResArgs<S, BSys> &a = args[k];
-    a = ResArgs<S, BSys>{};
+    Args &a = *new (&args[k]) Args{};
     a.n = q.n;
     a.grid = (q.n + c.rows - 1) / c.rows;
     a.rows = (q.n + a.grid - 1) / a.grid;
     a.first = wg;
+    std::fill(owner + wg, owner + wg + a.grid, (int)k);
     wg += a.grid;
     a.m[0] = ResCsr<S>{q.rowptr, q.col, q.g, q.c, q.sig_re, q.sig_im};
     a.inv = sys[k].inv;
@@ -146,12 +150,9 @@ ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S
     a.slots = a.words + (a.grid > 1 ? (size_t)kVecs * q.n * Tagged<S>::kWords : 0);
     a.outcome = a.slots + (size_t)2 * a.grid * kResSlotWords;
   }
-  ResArgs<S, BSys> *d_args = reinterpret_cast<ResArgs<S, BSys> *>(static_cast<char *>(ws) + args_at);
-  int *d_owner = reinterpret_cast<int *>(static_cast<char *>(ws) + owner_at);
-  OHM_HIP(hipMemcpyAsync(d_args, args.data(), sizeof(args[0]) * args.size(), hipMemcpyHostToDevice,
-                         b->stream));
-  OHM_HIP(hipMemcpyAsync(d_owner, owner.data(), sizeof(int) * owner.size(), hipMemcpyHostToDevice,
-                         b->stream));
+  Args *d_args = reinterpret_cast<Args *>(static_cast<char *>(ws) + args_at);
+  int *d_owner = reinterpret_cast<int *>(static_cast<char *>(ws) + args_at + owner_off);
+  OHM_HIP(hipMemcpyAsync(d_args, tables.data(), tables.size(), hipMemcpyHostToDevice, b->stream));
   hipLaunchKernelGGL(k_clear_words, dim3(grid_for((int64_t)words)), dim3(kBlock), 0, b->stream,
                      (int64_t)words, base);
   b->dispatches++;
@@ -182,8 +183,9 @@ template bool batch_resident_fits<double>(const ohm_backend *,
 template bool batch_resident_fits<cx<double>>(const ohm_backend *,
                                               const std::vector<BatchSolve<cx<double>>> &);
 template ohm_status batch_resident_enqueue<double>(ohm_backend *,
-                                                   const std::vector<BatchSolve<double>> &);
+                                                   const std::vector<BatchSolve<double>> &,
+                                                   std::vector<char> &);
 template ohm_status batch_resident_enqueue<cx<double>>(
-    ohm_backend *, const std::vector<BatchSolve<cx<double>>> &);
+    ohm_backend *, const std::vector<BatchSolve<cx<double>>> &, std::vector<char> &);
 
 }  // namespace ohm
