@@ -49,7 +49,6 @@ struct BBlock {
   int slot;  // position in the full block table: partial-sum slot
 };
 
-constexpr int kPersistRows = 4096;  // systems this small run in the persistent kernel
 constexpr int kBatchPartials = 5;   // most partial sums one reduction writes
 
 // Sum K values over the workgroup for one system; the last block of the
@@ -860,6 +859,7 @@ struct ohm_batch {
   std::vector<void *> allocs;    // patterns and values
   std::vector<int64_t> h_nnz;    // per system
   std::vector<int> h_long;       // per system: rows with more than 4, 6 and 8 entries
+  std::vector<int> h_scatter;    // per system: scattered_lines
   std::vector<char> res_tables;  // of the resident solve under way, while they upload
   bool has_f32 = false;
   bool jac64_valid = false, jac32_valid = false;  // Jacobi inverses match the current sigmas
@@ -1033,7 +1033,7 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
     for (int k = 0; k < K; k++)
       if (run[k] && bt->h_geo[k].n > 0) {
         const int64_t off = bt->h_geo[k].off;
-        list.push_back({&bt->h_geo[k], &bt->h_long[3 * (size_t)k], w.x + off, w.r + off, w.rh + off,
+        list.push_back({&bt->h_geo[k], &bt->h_long[3 * (size_t)k], bt->h_scatter[k], w.x + off, w.r + off, w.rh + off,
                         pk == PK_JACOBI ? w.inv + off : nullptr, bt->d_sys + k});
       }
     if (o.check_interval <= 0 && batch_resident_fits<S>(b, list)) {
@@ -1523,6 +1523,7 @@ ohm_status ohm_batch_create(ohm_backend *b, int32_t is_complex, int64_t k,
     int lr[3] = {0, 0, 0};
     if (n > 0) count_long_rows(q.rowptr, n, lr);
     bt->h_long.insert(bt->h_long.end(), lr, lr + 3);
+    bt->h_scatter.push_back(n > 0 ? scattered_lines(q.rowptr, q.col, n) : 0);
     host_rowptr.push_back(q.rowptr);
     bt->max_n = std::max(bt->max_n, n);
     off += n;

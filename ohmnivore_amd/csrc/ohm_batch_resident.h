@@ -13,13 +13,14 @@ template <typename S>
 struct BatchSolve {
   const BGeo *geo;
   const int *long_rows;   // rows with more than 4, 6 and 8 entries
+  int scatter;            // scattered_lines of its pattern
   S *x;
   const S *r, *rh, *inv;  // inv null: no preconditioner
   BSys *st;
 };
 
 // Whether these systems take the resident path: their workgroups run at once
-// in at most kResBatchGroups launches.
+// in one launch or two, and that is faster than the batch engine's own kernels.
 template <typename S>
 bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys);
 

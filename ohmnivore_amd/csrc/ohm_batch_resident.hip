@@ -11,8 +11,8 @@
 //
 // Bound, as there, by the latency of its reductions and by registers (complex
 // tiles of six entries spill). Systems that do not fit the chip together go in
-// groups, one launch after another; with more than kResBatchGroups of them the
-// nine launches, or a workgroup per system, do as well. Measured, ten
+// two launches, one after the other; with more the nine launches, or a workgroup
+// per system, do as well. Measured, ten
 // backward-Euler steps of 8 x 16,388 real rows 39.7 -> 15.0 ms (1,150
 // iterations); 21 x 1,847 complex rows 16.6 -> 7.3 ms (375 to 481 iterations).
 #include <algorithm>
@@ -27,7 +27,6 @@ namespace ohm {
 // enough without requests ahead of a reduction. Complex: eight waves, 256.
 template <typename S>
 constexpr int kResBatchRows = Tr<S>::C ? 512 : 640;
-constexpr int kResBatchGroups = 2;
 
 template <typename S, int W>
 __global__ __launch_bounds__(kResBatchRows<S>) void k_batch_resident(
@@ -59,27 +58,54 @@ struct Cut {
 };
 
 // Rows per workgroup, tile width and launches of a list of systems; rows == 0
-// when it does not fit.
+// when it does not fit, or where the batch engine's own kernels (a workgroup per
+// system up to kPersistRows, else nine launches per iteration) are as fast. Those
+// cost 7 to 10 us an iteration up to 500 rows, 16 (complex 19) at 1,024, 28 (34)
+// at 2,025, 52 (64) at 4,096 and about 37 beyond; here it is, per launch, 5 to 7 us
+// with one workgroup a system and 10 to 15 with several, complex 10 to 30.
 template <typename S>
 Cut cut_batch(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
   Cut c;
+  constexpr bool cplx = Tr<S>::C;
+  int most = 0, places = 0;
+  int64_t total = 0;
+  for (const auto &s : sys) {
+    most = std::max(most, s.geo->n);
+    total += s.geo->n;
+    places = std::max(places, s.scatter);
+  }
+  // whole solves, own kernels -> here: 9 real rows 131 -> 147 us, 25 179 -> 151;
+  // complex 256 rows 414 -> 538 us, 1,024 1,281 -> 1,300, 1,225 1,459 -> 1,274
+  if (most < (cplx ? 1025 : 24)) return c;
+  // in random order, complex: a mesh of 1,225 rows 1,581 -> 1,991 us, 2,025 2,442
+  // -> 2,270, 16,384 2,250 -> 2,408; a ladder of 1,100 about even, 1,700 1,900 ->
+  // 1,627, 16,384 2,961 -> 1,849, four of 30,000 3,311 -> 3,755
+  if (cplx && places > 40 &&
+      (most < 1600 || (most > kPersistRows && (places > 185 || total > 50'000))))
+    return c;
   static const int kWidths[3] = {4, 6, 8};
+  int longs = 0;
   for (int w = 0; w < 3 && !c.width; w++) {
-    bool fits = true;
-    for (const auto &s : sys) fits = fits && s.long_rows[w] <= kResMaxLong;
-    if (fits) c.width = kWidths[w];
+    longs = 0;
+    for (const auto &s : sys) longs = std::max(longs, s.long_rows[w]);
+    if (longs <= kResMaxLong) c.width = kWidths[w];
   }
   if (!c.width) return c;
+  // 3 to 4 us (complex 4 to 5) per long row: real, two of them, 83 rows 328 ->
+  // 355 us, 227 474 -> 484, 258 536 -> 443; 678 947 -> 1,108, 786 1,083 -> 1,033
+  const bool one_wg = most <= kResBatchRows<S>;
+  if (longs && cplx && most < 1400) return c;
+  if (longs > 1 && !cplx && (most <= 256 || (!one_wg && most < 768))) return c;
   const int cus = std::min(b->num_cu, kResMaxGrid);
-  // the smallest workgroups that need the fewest launches; systems of one
-  // workgroup each wait for nobody, so any number of them shares a launch
+  // Systems of one workgroup each wait for nobody, so any number of them
+  // shares a launch; else the smallest workgroups that need the fewest launches.
   for (int rows : {256, 320, 384, 448, 512, 576, 640}) {
     if (rows > kResBatchRows<S>) break;
+    if (one_wg && rows < most) continue;
     std::vector<int> group(1, 0);
     int used = 0;
-    bool fits = true, waits = false;
-    for (const auto &s : sys) waits = waits || s.geo->n > rows;
-    for (size_t k = 0; waits && k < sys.size(); k++) {
+    bool fits = true;
+    for (size_t k = 0; most > rows && k < sys.size(); k++) {
       const int wgs = (sys[k].geo->n + rows - 1) / rows;
       fits = fits && wgs <= cus;
       if (used > 0 && used + wgs > cus) {
@@ -94,7 +120,13 @@ Cut cut_batch(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
       c.group = group;
     }
   }
-  if (c.rows && (int)c.group.size() - 1 > kResBatchGroups) c.rows = 0;
+  // two launches: real, 144 x 1,024 rows 1,208 -> 1,525 us, 163 x 1,225 1,597 ->
+  // 1,584, 16 x 12,100 2,656 -> 1,793, 4 x 60,000 with two random neighbours a row
+  // 1,466 -> 1,616; complex 68 x 2,116 3,003 -> 3,323, 45 x 3,249 4,281 -> 3,503,
+  // 12 x 12,100 2,859 -> 3,676
+  const int groups = (int)c.group.size() - 1;
+  const bool two = places <= 40 && (cplx ? most > 2600 && most <= kPersistRows : most >= 1200);
+  if (groups > (two ? 2 : 1)) c.rows = 0;
   return c;
 }
 

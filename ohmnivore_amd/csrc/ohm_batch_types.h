@@ -7,6 +7,10 @@
 
 namespace ohm {
 
+// Batches whose largest system has at most this many rows may run one
+// workgroup per system (k_bpersist).
+constexpr int kPersistRows = 4096;
+
 // ------------------------------------------------------------ scalars ----
 template <typename R>
 struct cx {

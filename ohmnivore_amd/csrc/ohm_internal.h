@@ -64,6 +64,7 @@ inline void with_per(int per, F &&f) {
   }
 }
 constexpr size_t kPinnedBytes = 512;     // host staging of status words
+constexpr int kScatterRows = 3500;       // single solves up to this size never ask how far rows read
 constexpr int64_t kDeferMaxReads = int64_t(1) << 21;  // consumer x producer workgroups re-summed
 
 // ----------------------------------------------------------- solve state --
@@ -117,7 +118,8 @@ struct DevCsr {
   int per = kSpmvNnzPerBlock / kBlock;  // entries per thread: tuned_nnz / kBlock
   // rows with more than 4, 6 and 8 entries, of A and of A^T (-1: not counted)
   int long_rows[3] = {-1, -1, -1}, t_long_rows[3] = {-1, -1, -1};
-  int scatter = 0, t_scatter = 0;  // scattered_lines of A and of A^T
+  // scattered_lines of A and of A^T; 0 up to kScatterRows rows
+  int scatter = 0, t_scatter = 0;
   std::vector<uint32_t> h_rowptr, h_col; // host copy of the pattern
   // small matrices: the one allocation that holds rowptr, col, val, diag_pos
   // and the first block table
@@ -193,10 +195,8 @@ int spmv_default_per(const uint32_t *rowptr, int n);
 void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]);
 // How many separate places 64 neighbouring rows read far from themselves:
 // groups of 8 columns outside the rows' own block of (nearly) 512, averaged over
-// eight samples; 0 up to kScatterRows rows, which no rule tells apart. Up to 20
-// for a mesh numbered row by row, 125 for a ladder and 250 for a mesh with
-// node numbers in random order.
-constexpr int kScatterRows = 3500;
+// eight samples. Up to 20 for a mesh numbered row by row, 125 for a ladder and
+// 250 for a mesh with node numbers in random order.
 int scattered_lines(const uint32_t *rowptr, const uint32_t *col, int n);
 // Pick the fastest (rows_cap, nnz_cap) for m by timing each candidate.
 // fused: m is applied by the fused BiCGSTAB kernels (keep 256-row blocks)

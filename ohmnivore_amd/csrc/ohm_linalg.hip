@@ -75,8 +75,8 @@ void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]) {
 }
 
 int scattered_lines(const uint32_t *rowptr, const uint32_t *col, int n) {
-  if (n <= kScatterRows) return 0;
   constexpr int kSamples = 8, kRows = 64, kBlockRows = 512;
+  if (n <= kBlockRows) return 0;
   const int blocks = (n + kBlockRows - 1) / kBlockRows, rows = (n + blocks - 1) / blocks;
   std::vector<uint32_t> lines;
   size_t total = 0;
@@ -281,7 +281,7 @@ ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32
   m.h_rowptr.assign(rowptr, rowptr + n + 1);
   m.h_col.assign(col, col + nnz);
   count_long_rows(rowptr, n, m.long_rows);
-  m.scatter = scattered_lines(rowptr, col, n);
+  m.scatter = n > kScatterRows ? scattered_lines(rowptr, col, n) : 0;
   std::vector<uint32_t> bounds;
   m.per = spmv_default_per(rowptr, n);
   m.tuned_nnz = m.per * kBlock;
@@ -357,7 +357,7 @@ ohm_status csr_ensure_transpose(ohm_backend *b, DevCsr &m) {
     }
   std::vector<uint32_t> bounds;
   count_long_rows(trp.data(), n, m.t_long_rows);
-  m.t_scatter = scattered_lines(trp.data(), tcol.data(), n);
+  m.t_scatter = n > kScatterRows ? scattered_lines(trp.data(), tcol.data(), n) : 0;
   build_spmv_blocks(trp.data(), n, bounds);
   m.t_n_blocks = (int)bounds.size() - 1;
   const std::vector<uint32_t> blocks = spmv_block_pairs(trp.data(), bounds);

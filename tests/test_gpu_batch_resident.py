@@ -90,3 +90,39 @@ def test_batch_resident_one_system_fails_alone(be):
     bt.solve(b[:700].repeat(1).tolist() * 3, params=solver.bicgstab_params(
         tolerance=1e-14, max_iterations=2), raise_on_failure=False)
     assert [r.iterations for r in bt.last_results] == [2, 2, 2]
+
+
+def launches(be, sizes, per_row, complex_, n_dense=0):
+    """Kernel launches of one batched solve, checked against the first LU."""
+    rng = np.random.default_rng(sizes[0])
+    systems, rhs = [], []
+    for k, n in enumerate(sizes):
+        m = system(n, per_row, n_dense, seed=n)
+        diag = np.repeat(np.arange(n), np.diff(m.row_pointers.astype(np.int64))) == m.col_indices
+        systems.append((m.row_pointers, m.col_indices, m.values, np.abs(m.values) * 0.1 * diag,
+                        1j if complex_ else 0.5))
+        rhs.append(rng.standard_normal(n) + (1j * rng.standard_normal(n) if complex_ else 0))
+    bt = solver.Batch(be, systems, complex_)
+    prm = solver.bicgstab_params(tolerance=1e-13, max_iterations=2000)
+    before = be.counters()[0]
+    x = bt.solve(np.concatenate(rhs), params=prm)
+    n = be.counters()[0] - before
+    ref = lu(m if len(sizes) == 1 else system(sizes[0], per_row, n_dense, seed=sizes[0]),
+             systems[0][3], systems[0][4], rhs[0])
+    assert np.abs(bt.split(x)[0] - ref).max() < 1e-11 * np.abs(ref).max()
+    return n
+
+
+# Small batches, above all complex ones, are faster in one workgroup of the
+# engine's own, which is one launch where the resident solve is four; so are
+# two long rows up to 256, and two launches of less than 1,200 rows a system.
+@pytest.mark.parametrize("sizes,per_row,complex_,n_dense,resident", [
+    ([23], 3, False, 0, False), ([24], 3, False, 0, True), ([640] * 3, 3, False, 0, True),
+    ([1024], 3, True, 0, False), ([1025, 9], 3, True, 0, True),
+    ([256], 3, False, 2, False), ([257], 3, False, 2, True), ([700], 3, False, 2, False),
+    ([1399], 3, True, 1, False), ([1400], 3, True, 1, True),
+    ([700] * 140, 3, False, 0, False), ([1200] * 90, 3, False, 0, True)],
+    ids=lambda v: str(v[:2]) + f"x{len(v)}" if isinstance(v, list) else None)
+def test_batch_path_by_size(be, sizes, per_row, complex_, n_dense, resident):
+    n = launches(be, sizes, per_row, complex_, n_dense)
+    assert (n > 5) == resident, n
