@@ -32,7 +32,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
-#include <memory>
+#include <optional>
 #include <tuple>
 #include <vector>
 
@@ -1036,13 +1036,16 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
         list.push_back({&bt->h_geo[k], &bt->h_long[3 * (size_t)k], bt->h_scatter[k], w.x + off, w.r + off, w.rh + off,
                         pk == PK_JACOBI ? w.inv + off : nullptr, bt->d_sys + k});
       }
-    if (o.check_interval <= 0 && batch_resident_fits<S>(b, list)) {
-      ResidentGuard guard(true);
-      enqueue_start<S>(bt, w, (int)tab.size(), ia);
-      OHM_TRY(batch_resident_enqueue<S>(b, list, bt->res_tables));
-      OHM_HIP(hipMemcpyAsync(bt->h_sys, bt->d_sys, sizeof(BSys) * K, hipMemcpyDeviceToHost,
-                             stream));
-      OHM_HIP(hipStreamSynchronize(stream));
+    const int wgs = o.check_interval <= 0 ? batch_resident_workgroups<S>(b, list) : 0;
+    if (wgs > 0) {
+      {
+        ResidentPass pass(b->device, wgs, b->num_cu);
+        enqueue_start<S>(bt, w, (int)tab.size(), ia);
+        OHM_TRY(batch_resident_enqueue<S>(b, list, bt->res_tables));
+        OHM_HIP(hipMemcpyAsync(bt->h_sys, bt->d_sys, sizeof(BSys) * K, hipMemcpyDeviceToHost,
+                               stream));
+        OHM_HIP(hipStreamSynchronize(stream));
+      }
       b->readbacks++;
       bool all = true;
       for (int k = 0; k < K; k++) all = all && !(run[k] && bt->h_sys[k].status == ST_RUNNING);
@@ -2451,7 +2454,8 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
     }
     SegWord *hw = reinterpret_cast<SegWord *>(b->h_pinned);
     *hw = SegWord{0, 0, 0, (int)n_rec, 0, 0, 0, t};
-    auto resident = std::make_unique<ResidentGuard>(true);  // the segment may hold resident solves
+    std::optional<ResidentPass> pass;
+    if (captured_resident(tr->cs)) pass.emplace(b->device, captured_resident(tr->cs), b->num_cu);
     if ((rc = OHM_HIP_STATUS(hipMemcpyAsync(tr->d_seg, hw, sizeof(SegWord), hipMemcpyHostToDevice,
                                        stream))) != OHM_OK ||
         (rc = OHM_HIP_STATUS(hipGraphLaunch(exec, stream))) != OHM_OK ||
@@ -2460,7 +2464,7 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
         (rc = OHM_HIP_STATUS(hipStreamSynchronize(stream))) != OHM_OK)
       return false;
     b->readbacks++;
-    resident.reset();
+    pass.reset();
     const SegWord w = *hw;
     for (int j = 0; j < w.steps; j++) {  // accepted steps: the host's own clock
       t = ts[j];

@@ -19,14 +19,15 @@ struct BatchSolve {
   BSys *st;
 };
 
-// Whether these systems take the resident path: their workgroups run at once
-// in one launch or two, and that is faster than the batch engine's own kernels.
+// The most workgroups of one launch, when these systems take the resident path:
+// they run at once in one launch or two, and that is faster than the batch
+// engine's own kernels. Else 0.
 template <typename S>
-bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys);
+int batch_resident_workgroups(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys);
 
 // Enqueues the solves. A system that could not finish stays RUNNING with its
-// vectors untouched. The caller holds the resident lock until the launches
-// are done, and keeps `tables`, which the upload may still be reading, until
+// vectors untouched. The caller holds a ResidentPass for their workgroups until
+// the launches are done, and keeps `tables`, which the upload may still be reading, until
 // it has waited for the stream.
 template <typename S>
 ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys,

@@ -133,8 +133,16 @@ Cut cut_batch(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
 }  // namespace
 
 template <typename S>
-bool batch_resident_fits(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
-  return !sys.empty() && cut_batch<S>(b, sys).rows > 0;
+int batch_resident_workgroups(const ohm_backend *b, const std::vector<BatchSolve<S>> &sys) {
+  if (sys.empty()) return 0;
+  const Cut c = cut_batch<S>(b, sys);
+  int most = 0;
+  for (size_t q = 0; c.rows && q + 1 < c.group.size(); q++) {
+    int wgs = 0;
+    for (int k = c.group[q]; k < c.group[q + 1]; k++) wgs += (sys[k].geo->n + c.rows - 1) / c.rows;
+    most = std::max(most, wgs);
+  }
+  return most;
 }
 
 template <typename S>
@@ -210,10 +218,10 @@ ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S
   return OHM_OK;
 }
 
-template bool batch_resident_fits<double>(const ohm_backend *,
-                                          const std::vector<BatchSolve<double>> &);
-template bool batch_resident_fits<cx<double>>(const ohm_backend *,
-                                              const std::vector<BatchSolve<cx<double>>> &);
+template int batch_resident_workgroups<double>(const ohm_backend *,
+                                               const std::vector<BatchSolve<double>> &);
+template int batch_resident_workgroups<cx<double>>(const ohm_backend *,
+                                                   const std::vector<BatchSolve<cx<double>>> &);
 template ohm_status batch_resident_enqueue<double>(ohm_backend *,
                                                    const std::vector<BatchSolve<double>> &,
                                                    std::vector<char> &);

@@ -973,13 +973,15 @@ static ohm_status bicg_core(ohm_backend *b, const DevCsr &a, const PrecondDev &p
     void *ws = w.resident;
     if (!ws) OHM_TRY(resident_ws(b, lay.bytes, &ws));
     if (!w.resident || lay.bytes <= w.resident_bytes) {
-      ResidentGuard guard(true);
-      OHM_TRY(bicg_start<T>(b, a, p, rhs, w, o, pp, nullptr, ws, lay.clear_words));
-      OHM_TRY(resident_enqueue<T>(b, a, p, geo, ws, w.v, w.st));
       StatusWord *h = reinterpret_cast<StatusWord *>(b->h_pinned);
-      OHM_HIP(hipMemcpyAsync(h, &w.st->status, sizeof(StatusWord), hipMemcpyDeviceToHost,
-                             b->stream));
-      OHM_HIP(hipStreamSynchronize(b->stream));
+      {
+        ResidentPass pass(b->device, geo.grid, b->num_cu);
+        OHM_TRY(bicg_start<T>(b, a, p, rhs, w, o, pp, nullptr, ws, lay.clear_words));
+        OHM_TRY(resident_enqueue<T>(b, a, p, geo, ws, w.v, w.st));
+        OHM_HIP(hipMemcpyAsync(h, &w.st->status, sizeof(StatusWord), hipMemcpyDeviceToHost,
+                               b->stream));
+        OHM_HIP(hipStreamSynchronize(b->stream));
+      }
       b->readbacks++;
       out.polls++;
       if (h->status != ST_RUNNING) {
@@ -1050,6 +1052,8 @@ void captured_free(CapturedSolve *c) {
 }
 
 const SolveState *captured_state(const CapturedSolve *c) { return c->st; }
+
+int captured_resident(const CapturedSolve *c) { return c->geo.grid; }
 
 ohm_status captured_enqueue(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
                             const PrecondDev &p, const double *rhs, const BicgOpts &o, int iters,

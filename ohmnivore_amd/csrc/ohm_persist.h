@@ -4,6 +4,7 @@
 
 #include "ohm_precond.h"
 #include "ohm_reduce.h"
+#include "ohm_resident_gate.h"
 
 namespace ohm {
 
@@ -49,21 +50,5 @@ ohm_status resident_ws(ohm_backend *b, size_t bytes, void **ws);
 template <typename T>
 ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p, const ResGeo &g,
                             void *ws, const BicgVecs<T> &v, SolveState *st);
-
-// One resident solve at a time per process: two that share the GPU could each
-// hold the compute units the other waits for.
-void resident_lock();
-void resident_unlock();
-struct ResidentGuard {
-  bool on;
-  explicit ResidentGuard(bool take) : on(take) {
-    if (on) resident_lock();
-  }
-  ~ResidentGuard() {
-    if (on) resident_unlock();
-  }
-  ResidentGuard(const ResidentGuard &) = delete;
-  ResidentGuard &operator=(const ResidentGuard &) = delete;
-};
 
 }  // namespace ohm

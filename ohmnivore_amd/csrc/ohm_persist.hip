@@ -42,12 +42,12 @@
 // (16,388), 29.8 -> 15.9 (32,404), 35.7 -> 19.1 (65,540), 45.4 -> 25.4 (129,604).
 //
 // All workgroups must run at once: the grid has at most one workgroup per
-// compute unit. A wait that lasts longer than kResLimit ends the kernel with
-// nothing written (the outcome word says so to the other workgroups) and the
-// host continues with the pipeline from the state that k_init left; so does a
-// solve that breaks down.
+// compute unit, and the device's gate lets solves run together only if they fit
+// together (ohm_resident_gate.h). A wait that lasts longer than kResLimit ends the
+// kernel with nothing written (the outcome word says so to the other workgroups)
+// and the host continues with the pipeline from the state that k_init left; so
+// does a solve that breaks down.
 #include <algorithm>
-#include <mutex>
 
 #include "ohm_resident_dev.h"
 
@@ -64,10 +64,6 @@ __global__ __launch_bounds__(kResThreads) void k_bicg_resident(ResArgs<T, SolveS
 }
 
 // ------------------------------------------------------------ host side --
-static std::mutex g_resident_mu;
-void resident_lock() { g_resident_mu.lock(); }
-void resident_unlock() { g_resident_mu.unlock(); }
-
 // One row per thread: with two or three rows a thread's state leaves the
 // registers, and the pipeline, whose launches then carry enough work, is
 // faster (ISAI at 160,004 rows: 59 us per iteration against 49, at 262,148 97

@@ -127,6 +127,8 @@ const SolveState *captured_state(const CapturedSolve *c);
 // While *stop is non-zero (stop may be null) the whole solve is a no-op and
 // its state reads ST_SKIPPED. A solve still RUNNING after `iters`
 // iterations is finished by captured_resume.
+// Workgroups of the resident solve that each of its solves is (0: the pipeline).
+int captured_resident(const CapturedSolve *c);
 ohm_status captured_enqueue(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
                             const PrecondDev &p, const double *rhs, const BicgOpts &o, int iters,
                             const int *stop);

@@ -3,6 +3,8 @@ against the LU of every system and against the batch engine's own kernels,
 which a check_interval of one's own selects: real and complex, one workgroup
 per system and several, uneven sizes, one and two groups, rows longer than a
 tile, no preconditioner."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -126,3 +128,29 @@ def launches(be, sizes, per_row, complex_, n_dense=0):
 def test_batch_path_by_size(be, sizes, per_row, complex_, n_dense, resident):
     n = launches(be, sizes, per_row, complex_, n_dense)
     assert (n > 5) == resident, n
+
+
+def test_batch_resident_from_several_threads(be):
+    """Batches of four threads, each with its own backend: two fill most of the
+    device and take turns, two small ones run beside them. Each gives the
+    answer it gives alone."""
+    jobs = []
+    for n, k in ((1300, 60), (1300, 50), (2000, 2), (700, 5)):
+        m = system(n, 5, 0, seed=n)
+        mine = solver.HipBackend()
+        bt = solver.Batch(mine, [(m.row_pointers, m.col_indices, m.values, None, 0.0)] * k, False)
+        jobs.append((mine, bt, np.random.default_rng(n + k).standard_normal(n * k)))
+    prm = solver.bicgstab_params(tolerance=1e-13, max_iterations=2000)
+    alone = [bt.solve(b, params=prm).tobytes() for _, bt, b in jobs]
+    out = [[] for _ in jobs]
+
+    def work(k):
+        for _ in range(8):
+            out[k].append(jobs[k][1].solve(jobs[k][2], params=prm).tobytes())
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert [set(o) for o in out] == [{x} for x in alone]
