@@ -1036,7 +1036,8 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
         list.push_back({&bt->h_geo[k], &bt->h_long[3 * (size_t)k], bt->h_scatter[k], w.x + off, w.r + off, w.rh + off,
                         pk == PK_JACOBI ? w.inv + off : nullptr, bt->d_sys + k});
       }
-    const int wgs = o.check_interval <= 0 ? batch_resident_workgroups<S>(b, list) : 0;
+    ResidentGate &gate = resident_gate(b->device);
+    const int wgs = o.check_interval <= 0 && gate.open() ? batch_resident_workgroups<S>(b, list) : 0;
     if (wgs > 0) {
       {
         ResidentPass pass(b->device, wgs, b->num_cu);
@@ -1049,6 +1050,9 @@ ohm_status core_solve(ohm_batch *bt, BW<S> &w, const std::vector<char> &run, con
       b->readbacks++;
       bool all = true;
       for (int k = 0; k < K; k++) all = all && !(run[k] && bt->h_sys[k].status == ST_RUNNING);
+      bool gave_up = false;
+      if (!all) OHM_TRY(batch_resident_gave_up<S>(b, (int)list.size(), bt->res_tables, gave_up));
+      gate.report(gave_up);
       if (all) return OHM_OK;
     }
   }
@@ -2416,6 +2420,8 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
         return false;
       }
     }
+    ResidentGate &gate = resident_gate(b->device);
+    if (captured_resident(tr->cs) && !gate.open()) return false;
     hipGraphExec_t exec = nullptr;
     for (auto &g : tr->segs)
       if (g.steps == S && g.iters == seg_iters) exec = g.exec;
@@ -2466,6 +2472,7 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
     b->readbacks++;
     pass.reset();
     const SegWord w = *hw;
+    if (captured_resident(tr->cs) && w.stop != 1) gate.report(false);
     for (int j = 0; j < w.steps; j++) {  // accepted steps: the host's own clock
       t = ts[j];
       st.steps_accepted++;

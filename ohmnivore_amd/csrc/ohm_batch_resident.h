@@ -33,4 +33,10 @@ template <typename S>
 ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S>> &sys,
                                   std::vector<char> &tables);
 
+// Whether one of the `n` systems of these tables gave up because a wait outlasted
+// its limit.
+template <typename S>
+ohm_status batch_resident_gave_up(ohm_backend *b, int n, const std::vector<char> &tables,
+                                  bool &gave_up);
+
 }  // namespace ohm

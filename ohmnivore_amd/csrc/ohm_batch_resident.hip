@@ -170,6 +170,7 @@ ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S
   u64 *base = static_cast<u64 *>(ws);
   Args *args = reinterpret_cast<Args *>(tables.data());
   int *owner = reinterpret_cast<int *>(tables.data() + owner_off);
+  const int absent = resident_absent();
   int wg = 0;
   for (size_t k = 0; k < sys.size(); k++) {
     const BGeo &q = *sys[k].geo;
@@ -186,6 +187,7 @@ ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S
     a.r = sys[k].r;
     a.rh = sys[k].rh;
     a.st = sys[k].st;
+    a.absent = absent;
     a.words = base + at[k];
     a.slots = a.words + (a.grid > 1 ? (size_t)kVecs * q.n * Tagged<S>::kWords : 0);
     a.outcome = a.slots + (size_t)2 * a.grid * kResSlotWords;
@@ -218,6 +220,15 @@ ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S
   return OHM_OK;
 }
 
+template <typename S>
+ohm_status batch_resident_gave_up(ohm_backend *b, int n, const std::vector<char> &tables,
+                                  bool &gave_up) {
+  const ResArgs<S, BSys> *args = reinterpret_cast<const ResArgs<S, BSys> *>(tables.data());
+  gave_up = false;
+  for (int k = 0; k < n && !gave_up; k++) OHM_TRY(resident_gave_up(b, args[k].outcome, gave_up));
+  return OHM_OK;
+}
+
 template int batch_resident_workgroups<double>(const ohm_backend *,
                                                const std::vector<BatchSolve<double>> &);
 template int batch_resident_workgroups<cx<double>>(const ohm_backend *,
@@ -227,5 +238,10 @@ template ohm_status batch_resident_enqueue<double>(ohm_backend *,
                                                    std::vector<char> &);
 template ohm_status batch_resident_enqueue<cx<double>>(
     ohm_backend *, const std::vector<BatchSolve<cx<double>>> &, std::vector<char> &);
+
+template ohm_status batch_resident_gave_up<double>(ohm_backend *, int, const std::vector<char> &,
+                                                   bool &);
+template ohm_status batch_resident_gave_up<cx<double>>(ohm_backend *, int,
+                                                       const std::vector<char> &, bool &);
 
 }  // namespace ohm

@@ -968,7 +968,8 @@ static ohm_status bicg_core(ohm_backend *b, const DevCsr &a, const PrecondDev &p
   Parts pp;
   constexpr bool f32 = std::is_same<T, float>::value;
   const ResGeo geo = resident_geometry(b, a, p, a.n, f32);
-  if (geo.grid && o.check_interval <= 0) {
+  ResidentGate &gate = resident_gate(b->device);
+  if (geo.grid && o.check_interval <= 0 && gate.open()) {
     const ResLayout lay = resident_layout(geo, p, a.n, f32);
     void *ws = w.resident;
     if (!ws) OHM_TRY(resident_ws(b, lay.bytes, &ws));
@@ -985,9 +986,13 @@ static ohm_status bicg_core(ohm_backend *b, const DevCsr &a, const PrecondDev &p
       b->readbacks++;
       out.polls++;
       if (h->status != ST_RUNNING) {
+        gate.report(false);
         bicg_out(h, out);
         return OHM_OK;
       }
+      bool gave_up = false;
+      OHM_TRY(resident_gave_up(b, static_cast<uint64_t *>(ws) + lay.outcome, gave_up));
+      gate.report(gave_up);
       // given up before any step: the pipeline takes the started solve over
       return bicg_drive<T>(b, a, p, w, o, pp, false, 0, out);
     }
@@ -1077,6 +1082,12 @@ ohm_status captured_resume(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
   hipLaunchKernelGGL(k_unskip, dim3(1), dim3(64), 0, b->stream, c->st);
   OHM_HIP(hipGetLastError());
   b->dispatches++;
+  if (c->geo.grid) {
+    bool gave_up = false;
+    const ResLayout l = resident_layout(c->geo, p, a.n, false);
+    OHM_TRY(resident_gave_up(b, static_cast<uint64_t *>(c->resident) + l.outcome, gave_up));
+    resident_gate(b->device).report(gave_up);
+  }
   return bicg_drive<double>(b, a, p, c->w, o, c->pp, true, enqueued, out);
 }
 

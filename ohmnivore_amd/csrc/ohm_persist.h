@@ -51,4 +51,12 @@ template <typename T>
 ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p, const ResGeo &g,
                             void *ws, const BicgVecs<T> &v, SolveState *st);
 
+// Whether the solve with this outcome word (on the device) ended because a wait
+// outlasted its limit; waits for the stream. For solves left RUNNING.
+ohm_status resident_gave_up(ohm_backend *b, const void *outcome, bool &gave_up);
+
+// OHM_RESIDENT_ABSENT=1 (tests): the last workgroup of every solve stays away, as
+// on a device that does not run it, and the others give up.
+int resident_absent();
+
 }  // namespace ohm

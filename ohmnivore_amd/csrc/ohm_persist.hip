@@ -48,6 +48,7 @@
 // and the host continues with the pipeline from the state that k_init left; so
 // does a solve that breaks down.
 #include <algorithm>
+#include <cstdlib>
 
 #include "ohm_resident_dev.h"
 
@@ -64,6 +65,19 @@ __global__ __launch_bounds__(kResThreads) void k_bicg_resident(ResArgs<T, SolveS
 }
 
 // ------------------------------------------------------------ host side --
+int resident_absent() {
+  const char *e = getenv("OHM_RESIDENT_ABSENT");
+  return e && atoi(e) != 0;
+}
+
+ohm_status resident_gave_up(ohm_backend *b, const void *outcome, bool &gave_up) {
+  u64 o = RES_OPEN;
+  OHM_HIP(hipMemcpyAsync(&o, outcome, sizeof(o), hipMemcpyDeviceToHost, b->stream));
+  OHM_HIP(hipStreamSynchronize(b->stream));
+  gave_up = o == RES_ABORT;
+  return OHM_OK;
+}
+
 // One row per thread: with two or three rows a thread's state leaves the
 // registers, and the pipeline, whose launches then carry enough work, is
 // faster (ISAI at 160,004 rows: 59 us per iteration against 49, at 262,148 97
@@ -207,6 +221,7 @@ ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p
   q.r = v.r;
   q.rh = v.rh;
   q.st = st;
+  q.absent = resident_absent();
   q.words = reinterpret_cast<u64 *>(base);
   q.slots = q.words + l.slots;
   q.outcome = q.words + l.outcome;

@@ -14,7 +14,8 @@ namespace ohm {
 typedef unsigned long long u64;
 
 constexpr u64 kResLimit = 20'000'000;  // 0.2 s of the 100 MHz wall clock
-enum : u64 { RES_OPEN = 0, RES_COMMIT = 1, RES_ABORT = 2 };
+// How a solve ended: it stands, a wait outlasted the limit, or it broke down.
+enum : u64 { RES_OPEN = 0, RES_COMMIT = 1, RES_ABORT = 2, RES_BROKE = 3 };
 
 // A matrix G + sigma C (c null: G alone).
 template <typename S>
@@ -42,6 +43,7 @@ struct ResArgs {
   St *st;
   u64 *words;                // tagged vectors: r, q, v, tmp, hat
   u64 *slots, *outcome;
+  int absent;                // the last workgroup stays away (resident_absent)
 };
 
 // Scalar algebra: 64-bit, complex where the vectors are.
@@ -157,7 +159,7 @@ __device__ __forceinline__ bool res_expired(u64 *outcome, volatile int *dead, u6
     }
     return false;
   }
-  if (o == RES_ABORT) {
+  if (o >= RES_ABORT) {
     *dead = 1;
     return true;
   }
@@ -754,7 +756,8 @@ struct Resident {
   __device__ __forceinline__ void solve() {
     if (t == 0) {
       sh.dead = 0;
-      sh.run = a.st->status == ST_RUNNING && res_load(a.outcome) == RES_OPEN;
+      sh.run = a.st->status == ST_RUNNING && res_load(a.outcome) == RES_OPEN &&
+               !(a.absent && G > 1 && g == G - 1);
 #pragma unroll
       for (int m = 0; m < kMats; m++) sh.n_long[m] = sh.kept[m] = 0;
     }
@@ -906,7 +909,7 @@ struct Resident {
       u64 o = RES_OPEN;
       if (g == 0) {
         u64 want = RES_OPEN;
-        const u64 end = broke ? RES_ABORT : RES_COMMIT;
+        const u64 end = broke ? RES_BROKE : RES_COMMIT;
         __hip_atomic_compare_exchange_strong(a.outcome, &want, end, __ATOMIC_RELAXED,
                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         o = want == RES_OPEN ? end : want;

@@ -4,6 +4,7 @@ which a check_interval of one's own selects: real and complex, one workgroup
 per system and several, uneven sizes, one and two groups, rows longer than a
 tile, no preconditioner."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -154,3 +155,30 @@ def test_batch_resident_from_several_threads(be):
     for t in threads:
         t.join()
     assert [set(o) for o in out] == [{x} for x in alone]
+
+
+@pytest.mark.parametrize("complex_", [False, True], ids=["real", "complex"])
+def test_batch_resident_that_gives_up(be, complex_, monkeypatch):
+    """A workgroup of each system stays away: after 0.2 s the others give up,
+    the systems come back as they were and the engine's own kernels solve them, bit for bit as when they are asked to."""
+    sizes = [1300, 1500, 1100]
+    m = {n: system(n, 5, 0, seed=n) for n in sizes}
+    bt = solver.Batch(be, [(m[n].row_pointers, m[n].col_indices, m[n].values, 0.1 * m[n].values,
+                            1j if complex_ else 0.5) for n in sizes], complex_)
+    b = np.random.default_rng(4).standard_normal(sum(sizes)) * (1 + 1j if complex_ else 1)
+    prm = dict(tolerance=1e-12, max_iterations=2000)
+    own = bt.solve(b, params=solver.bicgstab_params(check_interval=8, **prm))
+    monkeypatch.setenv("OHM_RESIDENT_ABSENT", "1")
+    try:
+        x = bt.solve(b, params=solver.bicgstab_params(**prm))
+        assert x.tobytes() == own.tobytes()
+        monkeypatch.delenv("OHM_RESIDENT_ABSENT")
+        before = be.counters()[0]
+        y = bt.solve(b, params=solver.bicgstab_params(**prm))
+        assert y.tobytes() == own.tobytes() and be.counters()[0] - before < 6  # not tried
+    finally:
+        time.sleep(1.05)
+    before = be.counters()[0]
+    z = bt.solve(b, params=solver.bicgstab_params(**prm))
+    assert be.counters()[0] - before > 5
+    assert np.abs(z - own).max() < 1e-10 * np.abs(own).max()

@@ -4,6 +4,8 @@ multi-kernel pipeline, which a check_interval of one's own selects, at the
 edges of its dispatch: one workgroup and several, a last workgroup of few
 rows, row tiles of 4, 6 and 8 entries, rows longer than a tile, no
 preconditioner, FP32 refinement, warm starts and breakdowns."""
+import time
+
 import numpy as np
 import pytest
 
@@ -248,3 +250,30 @@ def test_more_than_two_long_rows_take_the_pipeline(be, prec):
         x, st = solve(be, a, b, prec, **TOL)
         assert np.abs(x - ref).max() < 1e-11 * np.abs(ref).max()
         assert (st.dispatches < 8) == resident
+
+
+@pytest.mark.parametrize("prec", [N.PREC_JACOBI, N.PREC_ISAI], ids=["jacobi", "isai"])
+def test_resident_solve_that_gives_up(be, prec, monkeypatch):
+    """One workgroup stays away: the others give the solve up when their first
+    wait has lasted 0.2 s, and the pipeline goes on from the start it left, to the
+    pipeline's own answer; the next solves leave the resident form out for a
+    second. Nothing is written by the solve that gave up: the warm start is
+    still there."""
+    n = 3000
+    a = system(n, 5, 0, seed=5)
+    b = np.random.default_rng(7).standard_normal(n)
+    ref = oracle.sparse_lu_solve(a, b)
+    x0 = ref + 1e-3 * np.random.default_rng(8).standard_normal(n)
+    pipe, sp = solve(be, a, b, prec, x0=x0, check_interval=8, **TOL)
+    monkeypatch.setenv("OHM_RESIDENT_ABSENT", "1")
+    try:
+        x, st = solve(be, a, b, prec, x0=x0, **TOL)
+        assert st.dispatches > 8 and st.iterations == sp.iterations
+        assert x.tobytes() == pipe.tobytes()
+        monkeypatch.delenv("OHM_RESIDENT_ABSENT")
+        _, later = solve(be, a, b, prec, x0=x0, **TOL)
+        assert later.dispatches > 8  # not tried
+    finally:
+        time.sleep(1.05)
+    _, again = solve(be, a, b, prec, x0=x0, **TOL)
+    assert again.dispatches < 8

@@ -1,5 +1,6 @@
 """The gate of the resident solves (host code, compiled here by itself): which
-solves run side by side on a device, and in which order they are let in."""
+solves run side by side on a device, in which order they are let in, and how
+long none is tried after one gave up."""
 import os
 import subprocess
 
@@ -51,6 +52,21 @@ int main() {
       }
     });
   for (auto &t : pool) t.join();
+  // a give-up closes the gate for 1, 2, 4 ... 32 s; a finished solve opens it
+  ResidentGate g;
+  int64_t now = 1000, want = 1000;
+  for (int k = 0; k < 8; k++) {
+    CHECK(g.open(now));
+    g.report(true, now);
+    CHECK(!g.open(now) && !g.open(now + want - 1) && g.open(now + want));
+    now += want;
+    want = want < 32000 ? 2 * want : want;
+    if (want > 32000) want = 32000;
+  }
+  g.report(false, now);
+  CHECK(g.open(now));
+  g.report(true, now);
+  CHECK(!g.open(now + 999) && g.open(now + 1000));
   std::printf("ok\n");
 }
 """
