@@ -116,11 +116,11 @@ def test_rc_grid_be_vs_oracle(be, precision):
 def test_captured_segments_match_eager(be, precond, monkeypatch):
     """Graph-captured BE timesteps (segments of up to 16 steps replayed as
     one graph, one segment-word read per segment) give bitwise the eager
-    loop's samples, final state and iteration counts; so do 3-step segments
-    whose 8 captured iterations per step are too few, so that every step
-    pauses and the host finishes its solve. Recording starts at tstart and
-    stops at max_records inside the segments."""
-    ckt = ir.rc_grid(24, 24, 12, seed=3)
+    loop's samples, final state and iteration counts; so do 3-step segments.
+    Recording starts at tstart and stops at max_records inside the segments.
+    The grid's solves are resident, one node each; those of
+    test_captured_pipeline_segments are iterations, which may be too few."""
+    ckt = early_sinks(ir.rc_grid(24, 24, 12, seed=3), 120e-12)
     mna = solver.compile(ckt)
     src, _ = T.source_table(ckt, mna)
     x0 = oracle.sparse_lu_solve(mna.g, mna.b_dc)
@@ -141,7 +141,59 @@ def test_captured_segments_match_eager(be, precond, monkeypatch):
                      r.steps_accepted, r.linear_solves, r.bicgstab_iterations)
     assert out["segments"] == out["eager"]
     assert out["paused"] == out["eager"]
+    assert out["eager"][5] > 120  # the sinks are on
     assert out["eager"][3] == 120 and len(np.frombuffer(out["eager"][0])) == 90
+
+
+def hub_grid():
+    """The 24 x 24 grid with three more nodes of twelve neighbours each: rows
+    too long for the resident solve, so that steps are solved by the pipeline."""
+    ckt = ir.rc_grid(24, 24, 12, seed=3)
+    nodes = [k for k in solver.compile(ckt).node_names if k != "0"]
+    for hub in range(3):
+        ckt.resistor(f"RH{hub}", f"hub{hub}", "0", 1e3)
+        ckt.capacitor(f"CH{hub}", f"hub{hub}", "0", 1e-13)
+        for k in range(12):
+            ckt.resistor(f"RH{hub}_{k}", f"hub{hub}", nodes[(41 * k + 17 * hub) % 570], 50.0 + k)
+    return ckt
+
+
+def early_sinks(ckt, t_end):
+    """The circuit's sinks, due within a nanosecond, switch on within t_end:
+    before that a step starts from its solution and takes no iterations."""
+    for w in ckt.tran.values():
+        w.td *= t_end / 1e-9
+    return ckt
+
+
+def run_segments(be, monkeypatch, ckt, steps, iters, precond, n_steps=120, **prm):
+    early_sinks(ckt, n_steps * 1e-12)
+    monkeypatch.setenv("OHM_TRAN_SEGMENT_STEPS", str(steps))
+    monkeypatch.setenv("OHM_TRAN_SEGMENT_ITERS", str(iters))
+    mna = solver.compile(ckt)
+    tr = T.Transient(be, mna, T.source_table(ckt, mna)[0])
+    x0 = oracle.sparse_lu_solve(mna.g, mna.b_dc)
+    before = be.counters()[1]
+    r = tr.run(1e-12, n_steps * 1e-12, method="be", x0=x0, precond=precond,
+               params=solver.bicgstab_params(tolerance=1e-12, **prm),
+               probes=np.arange(0, mna.size, 50))
+    return r, be.counters()[1] - before
+
+
+@pytest.mark.parametrize("precond", [N.PREC_ISAI, N.PREC_JACOBI], ids=["isai", "jacobi"])
+def test_captured_pipeline_segments(be, precond, monkeypatch):
+    """Segments whose captured solves are pipeline iterations: 16 steps with
+    enough of them cost one read each, 3-step segments with 8 iterations, too
+    few, pause at every step for the host to finish its solve. Both are bitwise
+    the eager loop."""
+    out = [run_segments(be, monkeypatch, hub_grid(), s, i, precond, max_iterations=20000)
+           for s, i in ((0, 0), (16, 160), (3, 8))]
+    for r, _ in out[1:]:
+        assert r.waves.tobytes() == out[0][0].waves.tobytes()
+        assert r.x_final.tobytes() == out[0][0].x_final.tobytes()
+        assert r.bicgstab_iterations == out[0][0].bicgstab_iterations > 120 * 8
+    reads = [n for _, n in out]
+    assert reads[1] < 40 and reads[2] > 2 * 110
 
 
 def test_breakdown_retried_inside_transient(be):
