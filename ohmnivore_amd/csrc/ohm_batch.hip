@@ -2411,7 +2411,10 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
       tt = tt + h;
       ts.push_back(tt);
     }
-    if (ts.size() < 2 || seg_iters > 256) return false;
+    // a resident solve is one node whatever its iterations
+    const bool one_node = resident_geometry(b, tr->A1, tr->P1, (int)tr->n, false).grid > 0;
+    const int budget = one_node ? 0 : seg_iters;
+    if (ts.size() < 2 || budget > 256) return false;
     const int S = (int)ts.size();
     if (!tr->cs) {
       if ((rc = captured_create(b, tr->A1, tr->P1, wx, &tr->cs)) != OHM_OK) return false;
@@ -2424,10 +2427,10 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
     if (captured_resident(tr->cs) && !gate.open()) return false;
     hipGraphExec_t exec = nullptr;
     for (auto &g : tr->segs)
-      if (g.steps == S && g.iters == seg_iters) exec = g.exec;
+      if (g.steps == S && g.iters == budget) exec = g.exec;
     if (!exec) {
       const int64_t saved = b->dispatches;
-      ohm_transient::SegGraph g{S, seg_iters, nullptr, nullptr};
+      ohm_transient::SegGraph g{S, budget, nullptr, nullptr};
       double *rhs = wx + 10 * stride;
       const int np = (int)n_probes;
       if ((rc = OHM_HIP_STATUS(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed))) != OHM_OK)
@@ -2442,7 +2445,7 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
                              order == 2 ? 2.0 : 1.0, order == 2 ? -1.0 : 0.0, wx, tr->d_save,
                              order == 2 ? tr->d_prev2 : (double *)nullptr, (double *)nullptr,
                              (const SegWord *)tr->d_seg);
-        rc = captured_enqueue(b, tr->cs, tr->A1, tr->P1, rhs, so, seg_iters, &tr->d_seg->stop);
+        rc = captured_enqueue(b, tr->cs, tr->A1, tr->P1, rhs, so, budget, &tr->d_seg->stop);
         hipLaunchKernelGGL(k_seg_close, dim3(1), dim3(64), 0, stream, tr->d_seg,
                            captured_state(tr->cs), h, tstart, (int)std::max<int64_t>(max_records, 0),
                            np, tr->d_probes, wx + bt->h_geo[0].off, tr->d_rec);
@@ -2491,7 +2494,7 @@ ohm_status ohm_transient_run(ohm_transient *tr, const double *x0, const ohm_tran
     if (w.stop == 1) {  // the step after the accepted ones needs more iterations
       BicgOut out;
       st.linear_solves++;
-      rc = captured_resume(b, tr->cs, tr->A1, tr->P1, so, seg_iters, out);
+      rc = captured_resume(b, tr->cs, tr->A1, tr->P1, so, budget, out);
       st.bicgstab_iterations += out.iters;
       if (rc == OHM_OK) rc = status_to_error(out.status, out.iters, so.max_iters);
       if (rc != OHM_OK) return false;

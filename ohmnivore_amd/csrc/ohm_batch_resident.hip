@@ -170,7 +170,7 @@ ohm_status batch_resident_enqueue(ohm_backend *b, const std::vector<BatchSolve<S
   u64 *base = static_cast<u64 *>(ws);
   Args *args = reinterpret_cast<Args *>(tables.data());
   int *owner = reinterpret_cast<int *>(tables.data() + owner_off);
-  const int absent = resident_absent();
+  const int absent = resident_absent(b);
   int wg = 0;
   for (size_t k = 0; k < sys.size(); k++) {
     const BGeo &q = *sys[k].geo;

@@ -1083,6 +1083,7 @@ ohm_status captured_resume(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
   OHM_HIP(hipGetLastError());
   b->dispatches++;
   if (c->geo.grid) {
+    enqueued = 0;  // given up, its one node has done nothing
     bool gave_up = false;
     const ResLayout l = resident_layout(c->geo, p, a.n, false);
     OHM_TRY(resident_gave_up(b, static_cast<uint64_t *>(c->resident) + l.outcome, gave_up));

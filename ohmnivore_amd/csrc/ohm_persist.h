@@ -56,7 +56,7 @@ ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p
 ohm_status resident_gave_up(ohm_backend *b, const void *outcome, bool &gave_up);
 
 // OHM_RESIDENT_ABSENT=1 (tests): the last workgroup of every solve stays away, as
-// on a device that does not run it, and the others give up.
-int resident_absent();
+// on a device that does not run it, and the others give up; 2: of captured ones.
+int resident_absent(const ohm_backend *b);
 
 }  // namespace ohm

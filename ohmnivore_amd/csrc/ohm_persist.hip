@@ -65,9 +65,12 @@ __global__ __launch_bounds__(kResThreads) void k_bicg_resident(ResArgs<T, SolveS
 }
 
 // ------------------------------------------------------------ host side --
-int resident_absent() {
+int resident_absent(const ohm_backend *b) {
   const char *e = getenv("OHM_RESIDENT_ABSENT");
-  return e && atoi(e) != 0;
+  const int v = e ? atoi(e) : 0;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (v == 2) (void)hipStreamIsCapturing(b->stream, &st);
+  return v == 1 || st != hipStreamCaptureStatusNone;
 }
 
 ohm_status resident_gave_up(ohm_backend *b, const void *outcome, bool &gave_up) {
@@ -221,7 +224,7 @@ ohm_status resident_enqueue(ohm_backend *b, const DevCsr &a, const PrecondDev &p
   q.r = v.r;
   q.rh = v.rh;
   q.st = st;
-  q.absent = resident_absent();
+  q.absent = resident_absent(b);
   q.words = reinterpret_cast<u64 *>(base);
   q.slots = q.words + l.slots;
   q.outcome = q.words + l.outcome;

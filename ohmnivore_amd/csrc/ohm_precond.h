@@ -122,20 +122,21 @@ ohm_status captured_create(ohm_backend *b, const DevCsr &a, const PrecondDev &p,
                            CapturedSolve **out);
 void captured_free(CapturedSolve *c);
 const SolveState *captured_state(const CapturedSolve *c);
+// Workgroups of the resident solve that each of its solves is (0: the pipeline).
+int captured_resident(const CapturedSolve *c);
 // Enqueues (no poll, no host decision) a solve of a x = rhs warm-started
 // from x: state reset, A x0, k_init, `iters` iterations and a closing check.
 // While *stop is non-zero (stop may be null) the whole solve is a no-op and
 // its state reads ST_SKIPPED. A solve still RUNNING after `iters`
-// iterations is finished by captured_resume.
-// Workgroups of the resident solve that each of its solves is (0: the pipeline).
-int captured_resident(const CapturedSolve *c);
+// iterations is finished by captured_resume. A resident solve is one node that
+// ignores `iters`; it stays RUNNING where it gave up or broke down.
 ohm_status captured_enqueue(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
                             const PrecondDev &p, const double *rhs, const BicgOpts &o, int iters,
                             const int *stop);
 // Drives an enqueued solve that was still RUNNING after its captured
 // iterations to its end (polls between chunks, as a plain solve does), also
-// after later masked-off solves on the same state; `enqueued` iterations
-// are already done.
+// after later masked-off solves on the same state. `enqueued`: the `iters` it was
+// captured with.
 ohm_status captured_resume(ohm_backend *b, CapturedSolve *c, const DevCsr &a,
                            const PrecondDev &p, const BicgOpts &o, int64_t enqueued,
                            BicgOut &out);

@@ -4,6 +4,7 @@ reference's adaptive TRAP/BE, FP64 and FP32 + FP64 refinement, one circuit
 and Monte Carlo instances. Tolerance 1e-6 relative / 1e-9 absolute per
 recorded sample."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -194,6 +195,35 @@ def test_captured_pipeline_segments(be, precond, monkeypatch):
         assert r.bicgstab_iterations == out[0][0].bicgstab_iterations > 120 * 8
     reads = [n for _, n in out]
     assert reads[1] < 40 and reads[2] > 2 * 110
+
+
+def test_resident_segments_ignore_the_iteration_budget(be, monkeypatch):
+    """A resident solve is one node, so a budget too long to capture does not
+    keep its steps out of a segment."""
+    (eager, n0), (seg, n1) = [
+        run_segments(be, monkeypatch, ir.rc_grid(24, 24, 12, seed=3), s, i, N.PREC_ISAI,
+                     max_iterations=20000) for s, i in ((0, 0), (16, 264))]
+    assert seg.waves.tobytes() == eager.waves.tobytes()
+    assert n0 >= 120 and n1 < 40
+
+
+def test_resident_segment_that_gives_up(be, monkeypatch):
+    """A captured resident solve that gives up has done no iterations: the host
+    drives it from its start with all of max_iterations left, whatever budget
+    the segment was captured with, and the steps after it are solved eagerly
+    for a second."""
+    eager, _ = run_segments(be, monkeypatch, ir.rc_grid(24, 24, 12, seed=3), 0, 0, N.PREC_ISAI,
+                            max_iterations=150)
+    monkeypatch.setenv("OHM_RESIDENT_ABSENT", "2")
+    try:
+        seg, reads = run_segments(be, monkeypatch, ir.rc_grid(24, 24, 12, seed=3), 16, 256,
+                                  N.PREC_ISAI, max_iterations=150)
+    finally:
+        time.sleep(1.05)
+    assert seg.steps_accepted == 120 and reads > 120
+    # steps solved to 1e-12 of the right-hand side by one path or the other
+    assert np.abs(seg.waves - eager.waves).max() < 1e-9 * np.abs(eager.waves).max()
+    assert np.abs(seg.x_final - eager.x_final).max() < 1e-9 * np.abs(eager.x_final).max()
 
 
 def test_breakdown_retried_inside_transient(be):
