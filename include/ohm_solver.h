@@ -309,7 +309,8 @@ ohm_status ohm_ac_plan_get_x(ohm_ac_plan *plan, int64_t circuit, int64_t f_first
  * whole one-lane LU when unpartitioned), residuals, one-lane redo of
  * systems whose partitioned residual exceeded 1e-12, unpermute; the rows
  * per part (0: one lane per whole system; picked by the autotuner on the
- * plan's first solve unless OHM_AC_PART_ROWS is set), the systems redone,
+ * plan's first solve, and kept for sweeps of about its size, unless
+ * OHM_AC_PART_ROWS is set), the systems redone,
  * and the chunks the sweep needed. Any pointer may be NULL. */
 ohm_status ohm_ac_plan_stats(const ohm_ac_plan *plan, double *phase_ms, int64_t *rows_per_part,
                              int64_t *fallback_systems, int32_t *chunks);

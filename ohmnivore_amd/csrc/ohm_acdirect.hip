@@ -1218,7 +1218,8 @@ struct ohm_ac_plan {
   uint64_t ws_gen = 0;
   std::vector<BandWave> waves;  // the resident chunk's wave table
   size_t y_off = 0;             // byte offset of its solutions in the workspace
-  int64_t tuned_rows = -1;      // autotuned rows per part (0: one lane per system)
+  int64_t tuned_rows = -1;      // autotuned rows per part (0: one lane per system),
+  int64_t tuned_from = 0;       // and default_part_rows of the sweep it was timed on
   bool tune = true;             // the autotuner may time candidates on this plan
   int64_t part_rows = 0;        // rows per part of the last solve
   int chunks = 0;
@@ -1797,7 +1798,7 @@ ohm_status plan_solve_once(ohm_ac_plan *p, int64_t n_freqs, double *const *x, in
 
 // rows per part: OHM_AC_PART_ROWS, else the autotuned value of this plan
 // (the fastest of the candidates, each timed over two whole sweeps on the
-// plan's first solve), else default_part_rows
+// plan's first solve) for sweeps like that one, else default_part_rows
 ohm_status plan_solve(ohm_ac_plan *p, int64_t n_freqs, const double *freqs, double *const *x,
                       ohm_batch_result *results, double *device_ms) {
   ohm_backend *b = p->b;
@@ -1828,11 +1829,14 @@ ohm_status plan_solve(ohm_ac_plan *p, int64_t n_freqs, const double *freqs, doub
   std::vector<double> omega(n_om, 0.0);
   for (int64_t f = 0; f < n_freqs; f++) omega[f] = 2.0 * M_PI * freqs[f];  // ac.rs:57
   OHM_HIP(hipMemcpyAsync(p->d_omega, omega.data(), sizeof(double) * n_om, hipMemcpyHostToDevice, st));
-  int64_t R = default_part_rows(p, n_freqs);
+  const int64_t rule = default_part_rows(p, n_freqs);
+  int64_t R = rule;
   if (const char *env = getenv("OHM_AC_PART_ROWS")) {
     R = atoll(env);
   } else if (p->tuned_rows >= 0) {
-    R = p->tuned_rows;
+    // timed on a sweep of one frequency a value says little about one of
+    // hundreds: it holds while the rule moves by half at most
+    if (2 * rule <= 3 * p->tuned_from && 2 * p->tuned_from <= 3 * rule) R = p->tuned_rows;
   } else if (b->autotune && p->tune && p->B == 1) {
     // each candidate timed twice (the faster of the two counts), so that a
     // sweep slowed by its first use of a workspace size does not decide
@@ -1852,6 +1856,7 @@ ohm_status plan_solve(ohm_ac_plan *p, int64_t n_freqs, const double *freqs, doub
       }
     }
     p->tuned_rows = R;
+    p->tuned_from = rule;
   }
   OHM_TRY(plan_solve_once(p, n_freqs, x, R));
   if (!p->h_final) {

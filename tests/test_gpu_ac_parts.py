@@ -52,3 +52,19 @@ def test_rows_per_part_rule(be, sections, n_freqs, rows, monkeypatch):
     st = plan.stats()
     assert st["rows_per_part"] == rows and st["redone_systems"] == 0
     assert float(res.residual_norms.max()) < 1e-12
+
+
+def test_tuned_rows_hold_for_sweeps_like_the_first(be, monkeypatch):
+    """A plan tuned on one frequency keeps its rows per part for sweeps of a few;
+    400 frequencies, where the rule says twice as many rows, take the rule's."""
+    monkeypatch.delenv("OHM_AC_PART_ROWS", raising=False)
+    mnas = [solver.compile(ir.rlc_ladder(4000, ir.SplitMix64(k))) for k in range(16)]
+    plan = solver.AcPlan(be, mnas)
+    rows = []
+    for n in (1, 3, 400, 2):
+        res = plan.solve(10.0 ** np.linspace(0.0, 9.0, n))
+        assert float(res.residual_norms.max()) < 1e-12
+        rows.append(plan.stats()["rows_per_part"])
+    # sqrt(3 x 12,002) and 16 x 12,002 x 400 / (64 x 3,072), up to multiples of 32
+    assert rows[0] in (0, 96, 192, 288, 384, 768)
+    assert rows[1] == rows[0] == rows[3] and rows[2] == 416
