@@ -297,8 +297,15 @@ bool newton_small_fits(const ohm_newton_ctx *c, const ohm_newton_params &prm) {
   if (prm.precision != OHM_PRECISION_FP64 || prm.bicgstab_max_iterations <= 0 ||
       !(prm.bicgstab_tolerance > 0.0) || !std::isfinite(prm.bicgstab_tolerance))
     return false;
+  // one thread walks devices that share nodes: with 800 of them the general
+  // path's saved launches no longer make up for it (14 unknowns, ISAI: 200
+  // diodes 2.4 -> 1.8 ms a run, 400 5.6 -> 5.4, 800 8.9 -> 9.5)
+  if (c->serial_diode && c->nd > 512) return false;
+  // 256 threads sweep the factors where the general path has 1,024: 62
+  // unknowns and 460 entries 4.2 -> 3.7 ms, 545 4.9 -> 5.0, 948 11.0 -> 12.2; 52
+  // and 422 3.4 -> 3.2, 511 4.2 -> 4.4; 32 and 736 4.6 -> 3.7
   IsaiView v;
-  if (c->P.kind == PK_ISAI && !isai_view(c->P, v)) return false;
+  if (c->P.kind == PK_ISAI && (!isai_view(c->P, v) || (c->n > 36 && v.nf > 448))) return false;
   return small_solve_lds(c) > 0;
 }
 

@@ -93,3 +93,52 @@ def test_small_newton_from_a_guess_and_after_an_update(be, monkeypatch):
     assert out["1"][:2] == out["0"][:2]
     # the adjoint's ILU sweeps start from factors of the run's last refresh
     assert np.allclose(out["1"][2], out["0"][2], rtol=1e-8, atol=1e-10 * np.abs(out["0"][2]).max())
+
+
+def random_mosfets(nodes, count, seed):
+    r = np.random.default_rng(seed)
+    c = ir.Circuit()
+    c.add_mosfet_model("M", vto=0.7, kp=1e-4, lam=0.02, nmos=True)
+    c.vsource("V1", "a", "0", dc=2.0)
+    for k in range(nodes):
+        c.resistor(f"R{k}", "a" if k == 0 else f"n{k - 1}", f"n{k}", 150.0)
+        c.resistor(f"S{k}", f"n{k}", "0", 1e4)
+    for k in range(count):
+        c.mosfet(f"M{k}", *(f"n{r.integers(nodes)}" for _ in range(3)), "M")
+    return c
+
+
+def shared_diodes(count):
+    c = ir.Circuit()
+    c.add_diode_model("D", 1e-14, 1.0)
+    c.vsource("V1", "a", "0", dc=2.0)
+    for k in range(8):
+        c.resistor(f"R{k}", "a" if k == 0 else f"n{k - 1}", f"n{k}", 150.0)
+    for k in range(count):
+        c.diode(f"D{k}", f"n{k % 8}", "0", "D")
+    return c
+
+
+# Where one workgroup is the slower one a run is the general path's: serial
+# limiting of many diodes, and large ISAI factors. Dense steps stay.
+@pytest.mark.parametrize("make,kw,small", [
+    (lambda: shared_diodes(512), dict(precond=N.PREC_ISAI), True),
+    (lambda: shared_diodes(513), dict(precond=N.PREC_ISAI), False),
+    (lambda: shared_diodes(513), dict(linear_solver="dense"), True),
+    (lambda: random_mosfets(58, 60, 1), dict(precond=N.PREC_ISAI), True),
+    (lambda: random_mosfets(58, 200, 1), dict(precond=N.PREC_ISAI), False),
+    (lambda: random_mosfets(58, 200, 1), dict(precond=N.PREC_JACOBI), True),
+    (lambda: random_mosfets(30, 900, 1), dict(precond=N.PREC_ISAI), True)],
+    ids=["512diodes", "513diodes", "513dense", "sparse", "dense_factors", "jacobi", "few_unknowns"])
+def test_small_newton_path_by_size(be, make, kw, small, monkeypatch):
+    m = solver.compile(make())
+    args = dict(abs_tol=1e-9, bicgstab_tolerance=1e-9, max_iterations=60, **kw)
+    monkeypatch.setenv("OHM_FUSED_SMALL", "1")
+    ctx = solver.NewtonContext(be, m.g, m.b_dc, m.diode_descriptors, m.bjt_descriptors,
+                               m.mosfet_descriptors)
+    ctx.run(**args)
+    before = be.counters()[0]
+    st = ctx.run(**args)
+    launches = be.counters()[0] - before
+    assert (launches < 4 * st.newton_iterations) == small, (launches, st.newton_iterations)
+    assert outcome(be, m, monkeypatch, True, **args) == outcome(be, m, monkeypatch, False, **args)
