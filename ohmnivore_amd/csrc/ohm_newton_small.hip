@@ -49,7 +49,7 @@ struct SmallArgs {
   IsaiView isai;
   SmallGather gm, gb;
   int serial_diode, serial_bjt;
-  int dense, first, budget, has_inv;
+  int dense, first, budget;
   double abs_tol, tol, floor_rel;
   int shadow, max_iters, scaled;
   Forcing fc;
