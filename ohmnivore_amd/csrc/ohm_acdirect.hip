@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <memory>
 #include <numeric>
@@ -1839,16 +1840,19 @@ ohm_status plan_solve(ohm_ac_plan *p, int64_t n_freqs, const double *freqs, doub
     if (2 * rule <= 3 * p->tuned_from && 2 * p->tuned_from <= 3 * rule) R = p->tuned_rows;
   } else if (b->autotune && p->tune && p->B == 1) {
     // each candidate timed twice (the faster of the two counts), so that a
-    // sweep slowed by its first use of a workspace size does not decide
+    // sweep slowed by its first use of a workspace size does not decide; by the
+    // clock, since more parts are also longer tables to make and upload (300
+    // circuits of 62 rows at 61 frequencies in parts of 32: 3 us less on the
+    // device, 60 us more in all)
     const int64_t cand[] = {0, R / 2, R, R + R / 2, 2 * R, 4 * R};
     double best = 1e300;
     for (int64_t c : cand) {
       double tc = 1e300;
       for (int rep = 0; rep < 2; rep++) {
+        const auto t0 = std::chrono::steady_clock::now();
         OHM_TRY(plan_solve_once(p, n_freqs, nullptr, c));
-        double t = 0.0;
-        for (double v : p->phase_ms) t += v;
-        tc = std::min(tc, t);
+        const std::chrono::duration<double> dt = std::chrono::steady_clock::now() - t0;
+        tc = std::min(tc, dt.count());
       }
       if (tc < best) {
         best = tc;

@@ -68,3 +68,15 @@ def test_tuned_rows_hold_for_sweeps_like_the_first(be, monkeypatch):
     # sqrt(3 x 12,002) and 16 x 12,002 x 400 / (64 x 3,072), up to multiples of 32
     assert rows[0] in (0, 96, 192, 288, 384, 768)
     assert rows[1] == rows[0] == rows[3] and rows[2] == 416
+
+
+def test_tuning_counts_the_host_side(be, monkeypatch):
+    """300 circuits of 62 rows: parts of 32 rows save a few us on the device and
+    cost 60 in tables, so the tuned plan has whole systems."""
+    monkeypatch.delenv("OHM_AC_PART_ROWS", raising=False)
+    ms = [solver.compile(ir.rlc_ladder(20, ir.SplitMix64(k))) for k in range(4)]
+    plan = solver.AcPlan(be, [ms[k % 4] for k in range(300)])
+    for _ in range(2):
+        res = plan.solve(10.0 ** np.linspace(0.0, 9.0, 61))
+    assert plan.stats()["rows_per_part"] == 0
+    assert float(res.residual_norms.max()) < 1e-12
