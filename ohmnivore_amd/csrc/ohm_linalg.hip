@@ -65,13 +65,16 @@ int spmv_default_per(const uint32_t *rowptr, int n) {
 }
 
 void count_long_rows(const uint32_t *rowptr, int n, int (&out)[3]) {
-  out[0] = out[1] = out[2] = 0;
+  int over4 = 0, over6 = 0, over8 = 0;  // and signed lengths: the loop runs in vectors
   for (int r = 0; r < n; r++) {
-    const uint32_t c = rowptr[r + 1] - rowptr[r];
-    out[0] += c > 4;
-    out[1] += c > 6;
-    out[2] += c > 8;
+    const int c = (int)(rowptr[r + 1] - rowptr[r]);
+    over4 += c > 4;
+    over6 += c > 6;
+    over8 += c > 8;
   }
+  out[0] = over4;
+  out[1] = over6;
+  out[2] = over8;
 }
 
 int scattered_lines(const uint32_t *rowptr, const uint32_t *col, int n) {
@@ -87,6 +90,8 @@ int scattered_lines(const uint32_t *rowptr, const uint32_t *col, int n) {
       const uint32_t lo = (uint32_t)(r / rows * rows);
       // a longer row's entries are read together
       const uint32_t end = std::min(rowptr[r + 1], rowptr[r] + 8);
+      // columns ascend: a row of its own block alone has nothing to add
+      if (end > rowptr[r] && col[rowptr[r]] >= lo && col[end - 1] - lo < (uint32_t)rows) continue;
       for (uint32_t k = rowptr[r]; k < end; k++)
         if (col[k] - lo >= (uint32_t)rows) lines.push_back(col[k] / 8);
     }
@@ -326,15 +331,19 @@ ohm_status csr_upload(ohm_backend *b, DevCsr &m, const double *val, const uint32
     }
     OHM_HIP(hipMemcpyAsync(m.pack, hold.data(), total, hipMemcpyHostToDevice, b->stream));
   } else {
-    // the tables made here are copied from `hold`, which outlives them
-    hold.resize(al(parts[3].bytes) + parts[4].bytes);
-    std::memcpy(hold.data(), parts[3].src, parts[3].bytes);
-    std::memcpy(hold.data() + al(parts[3].bytes), parts[4].src, parts[4].bytes);
+    // a caller that does not wait here keeps the tables made here
+    const void *srcs[5] = {parts[0].src, parts[1].src, parts[2].src, parts[3].src, parts[4].src};
+    if (stage) {
+      hold.resize(al(parts[3].bytes) + parts[4].bytes);
+      for (int k = 3; k < 5; k++) {
+        char *at = hold.data() + (k == 3 ? 0 : al(parts[3].bytes));
+        std::memcpy(at, parts[k].src, parts[k].bytes);
+        srcs[k] = at;
+      }
+    }
     for (const Part &p : parts) {
       OHM_HIP(hipMalloc(p.dev, p.bytes));
-      const void *src = &p == &parts[3]   ? hold.data()
-                        : &p == &parts[4] ? hold.data() + al(parts[3].bytes)
-                                          : p.src;
+      const void *src = srcs[&p - parts];
       if (p.copy) OHM_HIP(hipMemcpyAsync(*p.dev, src, p.copy, hipMemcpyHostToDevice, b->stream));
     }
   }

@@ -162,8 +162,11 @@ int resident_halo_rows(const ohm_backend *b, const DevCsr &a, const DevCsr &ml, 
       const uint32_t lo = (uint32_t)g * even, hi = (uint32_t)std::min(n, (g + 1) * even);
       list.clear();
       const auto join = [&](const DevCsr &m, uint32_t r, bool hat) {
-        if (!tile(m, r)) return;
-        for (uint32_t k = m.h_rowptr[r]; k < m.h_rowptr[r + 1]; k++) {
+        const uint32_t k0 = m.h_rowptr[r], k1 = m.h_rowptr[r + 1];
+        if (k0 == k1 || !tile(m, r)) return;
+        // columns ascend: most rows are done with their first and last
+        if (m.h_col[k0] >= lo && m.h_col[k1 - 1] < hi) return;
+        for (uint32_t k = k0; k < k1; k++) {
           const uint32_t c = m.h_col[k];
           if ((c >= lo && c < hi) || seen[c] == g || !tile(ml, c) || (hat && !tile(mu, c))) continue;
           seen[c] = g;
