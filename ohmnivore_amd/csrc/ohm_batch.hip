@@ -25,7 +25,9 @@
 // exit at their first instruction, and the host drops them from the table
 // when it polls (compaction), so converged frequency points stop costing
 // bandwidth. Systems of at most kPersistRows rows run instead in one
-// persistent launch with one workgroup per system iterating to convergence.
+// persistent launch with one workgroup per system iterating to convergence;
+// batches for which resident workgroups are faster than either go there
+// (cut_batch in ohm_batch_resident.hip).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

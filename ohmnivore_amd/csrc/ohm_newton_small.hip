@@ -11,11 +11,11 @@
 // the same order), so iterates and counts are its own to the bit.
 //
 // Bound by latency in one CU: the sub-solve's wave (7.8 us per BiCGSTAB
-// iteration at 54 unknowns) and the chains of the ILU / ISAI sweeps. Up to 64 unknowns, where
-// the one-wave solve applies: the rest of the chip would be idle either way.
-// 50-stage inverter chain .DC (390 Newton iterations in 39 runs) 75 -> 32-46 ms,
-// 20-stage .TRAN (1,229 iterations) 177 -> 96 ms: 76 us per ISAI iteration of
-// the former's 136, 60 per dense one.
+// iteration at 54 unknowns) and the chains of the ILU / ISAI sweeps. Up to 64
+// unknowns, where the one-wave solve applies (newton_small_fits has the other
+// bounds): the rest of the chip would be idle either way. 50-stage inverter
+// chain .DC (390 Newton iterations in 39 runs) 75 -> 31 ms, 20-stage .TRAN
+// (1,229 iterations) 177 -> 95 ms; 76 us per ISAI iteration, 60 per dense one.
 #include <algorithm>
 
 #include "ohm_dense_dev.h"

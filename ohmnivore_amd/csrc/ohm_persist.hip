@@ -38,8 +38,9 @@
 // workgroups, 1.2 us an exchange, 0.4 us a product from LDS and 0.8 us of
 // 64-bit scalar arithmetic. Measured per iteration, pipeline -> here: Jacobi
 // 15.3 -> 3.8 us (102 rows, one workgroup), 21.2 -> 9.7 (10,002), 21.7 -> 12.2
-// (65,540), 25.3 -> 15.8 (129,604); ISAI 29.3 -> 12.5 (2,871), 27.9 -> 15.1
+// (65,540), 25.3 -> 15.8 (129,604); ISAI 29.3 -> 12.1 (2,871), 27.9 -> 15.1
 // (16,388), 29.8 -> 15.9 (32,404), 35.7 -> 19.1 (65,540), 45.4 -> 25.4 (129,604).
+// Systems that lose by it are told apart in resident_geometry.
 //
 // All workgroups must run at once: the grid has at most one workgroup per
 // compute unit, and the device's gate lets solves run together only if they fit
