@@ -1527,12 +1527,19 @@ ohm_status ohm_batch_create(ohm_backend *b, int32_t is_complex, int64_t k,
       }
     }
     g.n_blocks = (int)bt->h_blocks.size() - g.first_block;
+    // systems of one pattern follow each other (the points of a sweep)
+    int lr[3] = {0, 0, 0}, places = 0;
+    if (s > 0 && bt->h_geo.back().rowptr == g.rowptr && bt->h_geo.back().n == n) {
+      std::copy(bt->h_long.end() - 3, bt->h_long.end(), lr);
+      places = bt->h_scatter.back();
+    } else if (n > 0) {
+      count_long_rows(q.rowptr, n, lr);
+      places = scattered_lines(q.rowptr, q.col, n);
+    }
+    bt->h_long.insert(bt->h_long.end(), lr, lr + 3);
+    bt->h_scatter.push_back(places);
     bt->h_geo.push_back(g);
     bt->h_nnz.push_back(nnz);
-    int lr[3] = {0, 0, 0};
-    if (n > 0) count_long_rows(q.rowptr, n, lr);
-    bt->h_long.insert(bt->h_long.end(), lr, lr + 3);
-    bt->h_scatter.push_back(n > 0 ? scattered_lines(q.rowptr, q.col, n) : 0);
     host_rowptr.push_back(q.rowptr);
     bt->max_n = std::max(bt->max_n, n);
     off += n;
